@@ -1234,6 +1234,107 @@ int qk_rope_impl(yx_ctx* c, yx_kv* kv, size_t layer, const yx::QkvIn& in, size_t
   return prof_end(c, YX_KERNEL_QK_ROPE, e0);
 }
 
+// Scratch of a matmul split along k: ks partial tiles of `elems` f32 per output tile and
+// one arrival counter per tile.
+int matmul_scratch(yx_ctx* c, size_t tiles, size_t ks, size_t elems) {
+  const size_t part = tiles * ks * elems * 4, cnt = tiles * 4 * yx::kCounterStride;
+  if (c->capturing && (c->mm_part.cap < part || c->mm_counters.cap < cnt))
+    return fail(YX_ERR_INVALID, "run the call once before capturing it (its scratch is allocated then)");
+  if (part > 0xffffffffu) return fail(YX_ERR_UNSUPPORTED, "matmul dimensions too large");
+  int rc;
+  if ((rc = c->mm_part.ensure(part, c->stream))) return rc;
+  return c->mm_counters.ensure(cnt, c->stream, true);
+}
+
+// At most 16 rows against many weight rows: the streaming kernel, for the k it is built
+// for (false: another one). From two 16-row tiles per CU on, where matmul_bf16_rows does
+// not split k (so the bits are the same): n 8192, k 2048 14.9 -> 10.5 us; at n 4096 8.9
+// against 10.0, but with k split the earlier kernel's sums are shorter (1.4e-7 against
+// 1.8e-7 off 64 bits), so it keeps those.
+// Tiles per batch: the count that leaves the busiest workgroup the fewest tiles, the
+// larger of equals (fewer barriers): n 151936 118 us with 2, 122 with 4, 128 with 8; n
+// 16384 15.0 with 4, 16.7 with 2.
+bool matmul_stream(yx_ctx* c, const float* x, const uint16_t* w, float* out, uint32_t t, uint32_t k, uint32_t n) {
+  if (k % 256) return false;
+  const uint32_t tiles = (n + 15) / 16, cus = static_cast<uint32_t>(c->cus);
+  uint32_t nb = 1, least = UINT32_MAX;
+  for (uint32_t b = 1; b <= static_cast<uint32_t>(yx::kStreamMaxBatch); b *= 2) {
+    const uint32_t batches = (tiles + b - 1) / b, busiest = (batches + cus - 1) / cus * b;
+    if (busiest <= least) {
+      least = busiest;
+      nb = b;
+    }
+  }
+  const dim3 grid(std::min(cus, (tiles + nb - 1) / nb));
+  const auto go = [&](auto* kern) {
+    hipLaunchKernelGGL(kern, grid, dim3(64 * yx::kStreamWaves), 0, c->stream, x, w, out, t, n, nb);
+    return true;
+  };
+  switch (k / 256) {
+    case 4: return go(yx::matmul_bf16_stream<4>);
+    case 6: return go(yx::matmul_bf16_stream<6>);
+    case 8: return go(yx::matmul_bf16_stream<8>);
+    case 10: return go(yx::matmul_bf16_stream<10>);
+    default: return false;
+  }
+}
+
+// Many rows: LDS tiles. The tile shape and the split of k with the smallest estimated
+// time: rounds of workgroups times a workgroup's time, its stages of 32 k times the
+// shape's cost per stage (all CUs busy, measured over t 20-4096, k 1536-3072, n
+// 2000-151936) plus start and output, plus a split's hand-off (its last workgroup reads
+// ks partial tiles at about 50 GB/s). The estimate picks
+// the fastest or one within 5% of it in those shapes (t 4096, n 2048: 128 x 256 tiles 87
+// us, 128 x 128 114, 64 x 128 123; t 512: 64 x 128 split in two 22.3, 128 x 128 in four
+// 22.9, 128 x 256 in two 45; t 80: 64 x 64 in four 12.0, 64 x 128 in eight 12.7).
+int matmul_tiled(yx_ctx* c, const float* x, const uint16_t* w, float* out, uint32_t t, uint32_t k, uint32_t n) {
+  struct Shape {
+    uint32_t tm, tn, per_cu;  // workgroups per CU
+    double stage_us;          // per 32 k, with per_cu workgroups on a CU
+  };
+  static constexpr Shape kShapes[] = {{128, 256, 1, 1.22}, {128, 128, 1, 0.75}, {64, 128, 1, 0.46}, {64, 64, 2, 0.56}};
+  const uint32_t steps = (k + 31) / 32;
+  int best = 0;
+  uint32_t best_ks = 1;
+  double best_us = 1e30;
+  for (int s = 0; s < 4; ++s) {
+    const Shape& sh = kShapes[s];
+    const uint64_t tiles = static_cast<uint64_t>((t + sh.tm - 1) / sh.tm) * ((n + sh.tn - 1) / sh.tn);
+    const uint64_t slots = static_cast<uint64_t>(sh.per_cu) * c->cus;
+    for (uint32_t ks = 1; ks <= 8 && (ks == 1 || (steps / ks >= 8 && tiles * ks <= slots)); ks *= 2) {
+      const uint64_t rounds = (tiles * ks + slots - 1) / slots;
+      // A CU with one workgroup where two fit runs it faster.
+      const double stage = tiles * ks * sh.per_cu <= slots ? sh.stage_us * 0.6 : sh.stage_us;
+      const double one = sh.per_cu == 1 ? sh.stage_us : stage;
+      const double us = 5.0 + rounds * (one * steps / ks + 1.0) + 
+                        (ks > 1 ? 1.0 + ks * (sh.tm * sh.tn) / 12500.0 : 0.0);
+      if (us < best_us) {
+        best_us = us;
+        best = s;
+        best_ks = ks;
+      }
+    }
+  }
+  const Shape& sh = kShapes[best];
+  const size_t tiles = static_cast<size_t>((t + sh.tm - 1) / sh.tm) * ((n + sh.tn - 1) / sh.tn);
+  if (tiles > 0x7fffffff) return fail(YX_ERR_UNSUPPORTED, "matmul dimensions too large");
+  int rc;
+  if (best_ks > 1 && (rc = matmul_scratch(c, tiles, best_ks, sh.tm * sh.tn))) return rc;
+  const auto go = [&](auto* kern) {
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(tiles), best_ks), dim3(yx::kMatmulThreads), 0, c->stream, x,
+                       w, out, t, k, n, static_cast<yx::f32x4*>(c->mm_part.p),
+                       static_cast<uint32_t>(c->mm_part.cap), static_cast<uint32_t*>(c->mm_counters.p));
+  };
+  switch (best) {
+    case 0: go(yx::matmul_bf16_tiles<yx::MatmulTileA>); break;
+    case 1: go(yx::matmul_bf16_tiles<yx::MatmulTileB>); break;
+    case 2: go(yx::matmul_bf16_tiles<yx::MatmulTileC>); break;
+    default: go(yx::matmul_bf16_tiles<yx::MatmulTileD>); break;
+  }
+  YX_HIP(hipGetLastError());
+  return YX_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1932,24 +2033,31 @@ int yx_matmul_bf16_dev(yx_ctx* c, const float* x, const uint16_t* w, float* out,
     return fail(YX_ERR_INVALID, "x and w must be 16-byte aligned");
   int rc = c->set_device();
   if (rc) return rc;
+  const size_t steps = (k + 31) / 32;
+  const auto T = static_cast<uint32_t>(t), K = static_cast<uint32_t>(k), N = static_cast<uint32_t>(n);
+  const size_t tiles16 = ((n + 15) / 16) * ((t + 15) / 16);
+  const size_t slots = static_cast<size_t>(c->cus);
+  if (c->matmul_k_split == 0 && tiles16 >= 2 * slots) {
+    if (t <= 16) {
+      if (matmul_stream(c, x, w, out, T, K, N)) {
+        YX_HIP(hipGetLastError());
+        return YX_OK;
+      }
+    } else if (k <= (size_t{1} << 20)) {  // a tile's rows within a buffer resource
+      return matmul_tiled(c, x, w, out, T, K, N);
+    }
+  }
   // Workgroups per output tile along k: about two workgroups per CU in all, each wave
   // at least one pass of its loop (kMmSteps steps of 32).
-  const size_t tiles = ((n + 15) / 16) * ((t + 15) / 16), steps = (k + 31) / 32;
-  size_t ks = std::max<size_t>(1, std::min<size_t>({(2 * static_cast<size_t>(c->cus) + tiles - 1) / tiles,
+  const size_t tiles = tiles16;
+  size_t ks = std::max<size_t>(1, std::min<size_t>({(2 * slots + tiles - 1) / tiles,
                                                      steps / (yx::kMmWaves * yx::kMmSteps), 64}));
   if (c->matmul_k_split > 0) ks = std::min<size_t>(static_cast<size_t>(c->matmul_k_split), steps);
-  if (ks > 1) {
-    if (c->capturing && (c->mm_part.cap < tiles * ks * 1024 || c->mm_counters.cap < tiles * 4 * yx::kCounterStride))
-      return fail(YX_ERR_INVALID, "run the call once before capturing it (its scratch is allocated then)");
-    if (tiles * ks * 1024 > 0xffffffffu) return fail(YX_ERR_UNSUPPORTED, "matmul dimensions too large");
-    if ((rc = c->mm_part.ensure(tiles * ks * 1024, c->stream))) return rc;
-    if ((rc = c->mm_counters.ensure(tiles * 4 * yx::kCounterStride, c->stream, true))) return rc;
-  }
+  if (ks > 1 && (rc = matmul_scratch(c, tiles, ks, 256))) return rc;
   hipLaunchKernelGGL(yx::matmul_bf16_rows,
                      dim3(static_cast<unsigned>((n + 15) / 16), static_cast<unsigned>((t + 15) / 16),
                           static_cast<unsigned>(ks)),
-                     dim3(64 * yx::kMmWaves), 0, c->stream, x, w, out, static_cast<uint32_t>(t),
-                     static_cast<uint32_t>(k), static_cast<uint32_t>(n),
+                     dim3(64 * yx::kMmWaves), 0, c->stream, x, w, out, T, K, N,
                      static_cast<yx::f32x4*>(c->mm_part.p), static_cast<uint32_t>(c->mm_part.cap),
                      static_cast<uint32_t*>(c->mm_counters.p));
   YX_HIP(hipGetLastError());

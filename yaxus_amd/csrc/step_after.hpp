@@ -3,7 +3,8 @@
 // 314-345: out[t][n] = x[t][:] . w[n][:], f32 activations, bf16 weight, f32 result) and
 // the greedy pick over logits (SyncReadback::argmax_rows, lib.rs:432-440, 556-558).
 //
-// matmul_bf16_rows: weight-bandwidth-bound for decode row counts. A workgroup owns 16
+// matmul_bf16_rows: for decode row counts against a projection's weight (other shapes:
+// matmul_bf16.hpp). A workgroup owns 16
 // output columns (weight rows) and 16 activation rows; its 8 waves take eighths of K and
 // their partial tiles are added in wave order (fixed, so the bits do not depend on
 // timing). Per 32 k, one v_mfma_f32_16x16x32_bf16 per part of x: the weight is bf16
@@ -27,12 +28,9 @@
 #include <stdint.h>
 
 #include "attn_decode.hpp"
+#include "matmul_bf16.hpp"
 
 namespace yx {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
 
 static constexpr int kMmWaves = 8;
 static constexpr int kMmSteps = 4;  // 32-wide k steps per wave and pass of its loop
