@@ -1,0 +1,45 @@
+"""Decode and verify passes of many sequences of different lengths: more work items than
+CUs, which the work list cuts into one round or dispatches longest first (all heads of an
+item in turn), against the oracle and against a split forced by an option."""
+
+import numpy as np
+import pytest
+
+from tests.scenario import D, Scenario, close
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("batch,rows,lo,hi,hq,hkv,page,window,f32", [
+    (70, 1, 200, 420, 8, 4, 16, 0, False),     # more (sequence, head) pairs than CUs: longest first
+    (66, 1, 1, 900, 16, 4, 32, 300, False),    # with a window, from one key on
+    (34, 1, 100, 1400, 16, 8, 128, 0, False),
+    (40, 3, 50, 1500, 16, 8, 16, 0, False),    # verify: two tiles
+    (18, 2, 300, 2600, 8, 4, 16, 0, False),
+    (70, 1, 100, 300, 8, 4, 16, 0, True),      # the f32 arena
+    (3, 1, 5000, 9000, 8, 1, 16, 0, False),
+])
+def test_ragged_pass(hip, batch, rows, lo, hi, hq, hkv, page, window, f32):
+    rng = np.random.default_rng(batch * 1000 + hi)
+    lens = [int(x) for x in np.exp(rng.uniform(np.log(lo), np.log(hi), batch))]
+    need = sum(-(-(n + rows) // page) for n in lens)
+    sc = Scenario(hip, pages=need + 8, page=page, hkv=hkv, pool_seed=batch, f32=f32)
+    try:
+        seqs = [sc.cache.new_seq() for _ in lens]
+        sc.prefill(dict(zip(seqs, lens)))
+        pr = sc.run_pass([(s, rows) for s in seqs])
+        t = len(pr.meta.pos)
+        k, v = (sc.draw(t * hkv * D).reshape(t, hkv, D) for _ in range(2))
+        q = sc.draw(t * hq * D).reshape(t, hq * D)
+        got = hip.attend_append(sc.kv, 0, k, v, q, hq, window=window)
+        again = hip.attend(sc.kv, 0, q, hq, window=window)
+        assert np.array_equal(got.view(np.uint32), again.view(np.uint32))
+        sc.orc[0].store(pr.meta.kv_slot, k.reshape(t, -1), v.reshape(t, -1))
+        want = sc.orc[0].attend(q, hq, pr.meta.pos, pr.meta.pt_off, pr.meta.pages, window=window)
+        assert close(got, want).all(), f"max abs err {np.abs(got - want).max()}"
+        hip.set_option("attn_max_chunk_blocks", 8)  # another split of the same keys
+        other = hip.attend(sc.kv, 0, q, hq, window=window)
+        assert np.abs(got - other).max() < 1e-5
+    finally:
+        hip.set_option("attn_max_chunk_blocks", 1 << 20)
+        sc.kv.destroy()

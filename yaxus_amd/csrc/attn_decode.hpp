@@ -727,10 +727,10 @@ __global__ __launch_bounds__(64 * kBalWaves) void paged_attn_decode_balanced(
     const float* __restrict__ knew, const float* __restrict__ vnew,
     const uint32_t* __restrict__ kv_slot, _Float16* kw, _Float16* vw,  // kw/vw alias kc/vc
     uint32_t part_o_bytes, uint32_t part_ml_bytes, uint32_t hq, uint32_t hkv,
-    uint32_t bpp_shift, uint32_t window, float scale_log2, QkvIn qi_in) {
+    uint32_t bpp_shift, uint32_t window, float scale_log2, QkvIn qi_in, uint32_t by_item) {
   __shared__ BalancedShared sh;
-  const AttnItem it = items[blockIdx.x];
-  const uint32_t kh = blockIdx.y;
+  const AttnItem it = items[by_item ? blockIdx.y : blockIdx.x];
+  const uint32_t kh = by_item ? blockIdx.x : blockIdx.y;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63;
   const int c = lane & 15, g = lane >> 4;
@@ -953,13 +953,13 @@ __global__ __launch_bounds__(64 * kWideWaves) void paged_attn_decode_wide(
     const uint32_t* __restrict__ kv_slot, _Float16* kw, _Float16* vw,  // kw/vw alias kc/vc
     uint32_t part_o_bytes, uint32_t part_ml_bytes, uint32_t hq, uint32_t hkv,
     uint32_t bpp_shift, uint32_t window, float scale_log2, QkvIn qi_in,
-    const SubRef* __restrict__ members) {
+    const SubRef* __restrict__ members, uint32_t by_item) {
   __shared__ WideShared<NT, false> sh;
   static_assert(sizeof(sh.o) >= (NT * 16 + kWideWaves) * kD * sizeof(float), "q and scratch fit");
   float (*const q_lds)[kD] = reinterpret_cast<float (*)[kD]>(&sh.o[0][0][0]);
   float* const qsq_lds = reinterpret_cast<float*>(&sh.o[0][0][0]) + NT * 16 * kD;
-  const AttnItem it = items[blockIdx.x];
-  const uint32_t kh = blockIdx.y;
+  const AttnItem it = items[by_item ? blockIdx.y : blockIdx.x];
+  const uint32_t kh = by_item ? blockIdx.x : blockIdx.y;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63;
   const int c = lane & 15, g = lane >> 4;
@@ -1229,10 +1229,11 @@ __global__ __launch_bounds__(64 * kWideWaves) void paged_attn_decode_f32(
     const float* __restrict__ knew, const float* __restrict__ vnew,
     const uint32_t* __restrict__ kv_slot, float* kw, float* vw,  // kw/vw alias kc/vc
     uint32_t part_o_bytes, uint32_t part_ml_bytes, uint32_t hq, uint32_t hkv,
-    uint32_t bpp_shift, uint32_t window, float scale_log2, const SubRef* __restrict__ members) {
+    uint32_t bpp_shift, uint32_t window, float scale_log2, const SubRef* __restrict__ members,
+    uint32_t by_item) {
   __shared__ WideShared<1, false> sh;
-  const AttnItem it = items[blockIdx.x];
-  const uint32_t kh = blockIdx.y;
+  const AttnItem it = items[by_item ? blockIdx.y : blockIdx.x];
+  const uint32_t kh = by_item ? blockIdx.x : blockIdx.y;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63;
   const int c = lane & 15, g = lane >> 4;

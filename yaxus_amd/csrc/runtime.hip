@@ -178,6 +178,7 @@ struct AttnPlan {
   DevBuf d_members;
   size_t cascades = 0;              // shared prefixes attended once for their groups
   bool fusable = false;  // the append can run inside the attention kernel
+  bool by_item = false;  // decode grid (hkv, items): items in list order, all heads of each in turn
   size_t slots = 0;     // partial slots (per kv head)
   size_t counters = 0;  // arrival counters (per kv head)
   bool uploaded = false;  // dev_items / dev_members hold the lists
@@ -771,13 +772,19 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
     if (tiny) cq = std::max<uint32_t>(cq, (nq + 7) / 8);
     return cq;
   };
+  // Bounds of chunk ch of nch of a group of nb blocks: on quads of blocks, or, where a
+  // chunk is too long for the queue kernel, on eights (the 16-row-tile kernel's waves
+  // then take equal shares of every chunk but the group's last).
+  auto chunk_begin = [&](uint32_t nb, uint32_t ch, uint32_t nch) {
+    const uint32_t unit = nb > nch * 4 * yx::kBalQuads ? yx::kWideWaves : 4, n = (nb + unit - 1) / unit;
+    return std::min(nb, unit * static_cast<uint32_t>(static_cast<uint64_t>(n) * ch / nch));
+  };
   // Whether every chunk's blocks split evenly over kWideWaves waves.
   auto exact_split = [&](size_t cbk) {
     auto check = [&](uint32_t nblocks) {
       const uint32_t nq = (nblocks + 3) / 4, cq = chunk_quads(nq, cbk), nch = (nq + cq - 1) / cq;
       for (uint32_t ch = 0; ch < nch; ++ch) {
-        const uint32_t b0 = 4 * static_cast<uint32_t>(static_cast<uint64_t>(nq) * ch / nch);
-        const uint32_t b1 = std::min(nblocks, 4 * static_cast<uint32_t>(static_cast<uint64_t>(nq) * (ch + 1) / nch));
+        const uint32_t b0 = chunk_begin(nblocks, ch, nch), b1 = chunk_begin(nblocks, ch + 1, nch);
         if ((b1 - b0) % yx::kWideWaves != 0) return false;
       }
       return true;
@@ -796,9 +803,101 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
   // 56-block minimums measured slower). Exact splits (the headline; B=8, ctx 4096) and
   // small passes keep one item per CU.
   constexpr size_t kMinItemBlocks = 40;
-  if (c->target_waves == 0 && nt == 1 && work >= static_cast<size_t>(c->cus) * kMinItemBlocks / 2 &&
+  if (!f32 && c->target_waves == 0 && nt == 1 && work >= static_cast<size_t>(c->cus) * kMinItemBlocks / 2 &&
       !exact_split(cb))
     cb = std::max<size_t>(cb, kMinItemBlocks);
+  // More work items than CUs (sequences of different lengths: each is cut into whole
+  // chunks of about the average load): a second, mostly empty round. Then the chunk
+  // length with the smallest estimated time: the shortest that gives at most one item
+  // per CU, or one near the average load with the items dispatched longest first. The
+  // estimate: the items' blocks, plus kStartBlocks per item (its start and hand-off, ~3
+  // us of a full GPU's 0.33 us per block and CU), dealt to the least loaded slot; the
+  // part above the average counts kTail, since the CUs still busy at the end share the
+  // bandwidth of the others (kStartBlocks 6-16 and kTail 0.35-0.9 measured: 10 instead
+  // of 16 is up to 11% slower, kTail hardly matters). Measured (us per layer, one item
+  // of the average load per CU and list order -> this): 48 sequences of 60-12000 keys,
+  // heads 24/4: 50.3 -> 42.2; 8 of 3169-11933, 16/8: 52.9 -> 41.5; 19 of 280-5543, 16/8:
+  // 38.2 -> 29.6; 30 of 2000-2100, 16/4: 38.4 -> 28.1; 5 of 16000-20000, 16/8: 84.2 ->
+  // 63.5; verify, 20 x 4 rows after 200-6000: 31.9 -> 22.2; f32, 20 of 200-9000, 16/8:
+  // 102.8 -> 78.8.
+  std::vector<uint32_t> lens;
+  auto estimate = [&](size_t cbk) {
+    constexpr uint32_t kStartBlocks = 16;
+    constexpr double kTail = 0.6;
+    lens.clear();
+    auto add = [&](uint32_t nb) {
+      const uint32_t nq = (nb + 3) / 4, cq = chunk_quads(nq, cbk), nch = (nq + cq - 1) / cq;
+      for (uint32_t ch = 0; ch < nch; ++ch)
+        lens.push_back(chunk_begin(nb, ch + 1, nch) - chunk_begin(nb, ch, nch) + kStartBlocks);
+    };
+    for (const Casc& cc : cascs) add(cc.blocks);
+    for (const Sub& sb : subs) add(sb.b1 - sb.b0);
+    std::sort(lens.begin(), lens.end(), std::greater<uint32_t>());
+    // Slots of one head: the heads' items are alike.
+    std::vector<uint32_t> load(std::max<size_t>(1, static_cast<size_t>(c->cus) / hkv), 0);
+    uint64_t total = 0;
+    uint32_t most = 0;
+    for (uint32_t n : lens) {  // min-heap of the slots' loads
+      std::pop_heap(load.begin(), load.end(), std::greater<uint32_t>());
+      load.back() += n;
+      most = std::max(most, load.back());
+      std::push_heap(load.begin(), load.end(), std::greater<uint32_t>());
+      total += n;
+    }
+    const double avg = static_cast<double>(total) / load.size();
+    return avg + kTail * (most - avg);
+  };
+  bool sort_items = false;
+  if (c->target_waves == 0) {
+    // Items of all heads; slots: those of groups in several chunks (a partial slot each).
+    auto items_of = [&](size_t cbk, size_t* slots = nullptr) {
+      size_t n = 0, sl = 0;
+      for (const Casc& cc : cascs) {
+        const uint32_t nq = (cc.blocks + 3) / 4, cq = chunk_quads(nq, cbk);
+        n += (nq + cq - 1) / cq;
+        sl += (nq + cq - 1) / cq;
+      }
+      for (const Sub& sb : subs) {
+        const uint32_t nq = (sb.b1 - sb.b0 + 3) / 4, cq = chunk_quads(nq, cbk), nch = (nq + cq - 1) / cq;
+        n += nch;
+        if (nch > 1 || sb.casc >= 0) sl += nch;
+      }
+      if (slots) *slots = sl * hkv;
+      return n * hkv;
+    };
+    const size_t cus = static_cast<size_t>(c->cus), limit = 64 * waves;
+    if (items_of(cb) > cus) {
+      const size_t avg = (work + cus - 1) / cus;
+      // Never more partials or items than the scratch of the entry point that allocates
+      // nothing holds, unless the plain split has more already.
+      size_t slots0;
+      const size_t items0 = items_of(cb, &slots0);
+      const size_t max_slots = std::max<size_t>(slots0, 640), max_items = std::max<size_t>(items0, 8192);
+      size_t best = cb;
+      double best_t = estimate(cb);
+      auto consider = [&](size_t cbk) {
+        cbk = std::min(std::max<size_t>(cbk, 16), limit);
+        size_t sl;
+        if (items_of(cbk, &sl) > max_items || sl > max_slots) return;
+        const double t = estimate(cbk);
+        if (t < best_t) {
+          best_t = t;
+          best = cbk;
+        }
+      };
+      if (items_of(limit) <= cus) {
+        size_t lo = cb, hi = limit;  // items_of(lo) > cus >= items_of(hi)
+        while (hi - lo > 4) {
+          const size_t mid = (lo + hi) / 2;
+          (items_of(mid) > cus ? lo : hi) = mid;
+        }
+        consider(hi);
+      }
+      for (size_t p : {60, 80, 100, 115, 135, 160}) consider(avg * p / 100);
+      cb = best;
+      sort_items = cascs.empty() && items_of(cb) > cus;
+    }
+  }
   // Each wave's page ids fit its 64 lanes: at most 64 blocks per wave.
   cb = std::max<size_t>(1, std::min<size_t>({cb, static_cast<size_t>(c->max_chunk_blocks), 64 * waves}));
 
@@ -833,8 +932,8 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
       w.r0 = cc.r0;
       w.nrows = cc.n;
       w.pt_off = cc.dev_off;
-      w.blk0 = 4 * static_cast<uint32_t>(static_cast<uint64_t>(nq) * ch / nch);
-      w.blk1 = std::min(cc.blocks, 4 * static_cast<uint32_t>(static_cast<uint64_t>(nq) * (ch + 1) / nch));
+      w.blk0 = chunk_begin(cc.blocks, ch, nch);
+      w.blk1 = chunk_begin(cc.blocks, ch + 1, nch);
       w.chunk = ch;
       w.nch = nch;
       w.part_base = static_cast<uint32_t>(slot);
@@ -859,8 +958,8 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
       w.r0 = s.r0;
       w.nrows = s.n;
       w.pt_off = s.dev_off;
-      w.blk0 = s.b0 + 4 * static_cast<uint32_t>(static_cast<uint64_t>(nq) * ch / nch);
-      w.blk1 = std::min(s.b1, s.b0 + 4 * static_cast<uint32_t>(static_cast<uint64_t>(nq) * (ch + 1) / nch));
+      w.blk0 = s.b0 + chunk_begin(s.b1 - s.b0, ch, nch);
+      w.blk1 = s.b0 + chunk_begin(s.b1 - s.b0, ch + 1, nch);
       w.chunk = ch;
       w.nch = nch;
       w.part_base = static_cast<uint32_t>(slot);
@@ -950,6 +1049,12 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
     for (const yx::AttnItem& w : plan.items)
       if ((w.blk1 - w.blk0) % yx::kWideWaves != 0) exact = false;
     plan.wide = !cascs.empty() || exact || !plan.balanced;
+  }
+  if (sort_items && plan.items.size() <= 0xffff) {
+    std::stable_sort(plan.items.begin(), plan.items.end(), [](const yx::AttnItem& a, const yx::AttnItem& b) {
+      return a.blk1 - a.blk0 > b.blk1 - b.blk0;
+    });
+    plan.by_item = plan.balanced || plan.wide;
   }
   plan.slots = slot;
   plan.counters = subs.size();
@@ -1111,6 +1216,8 @@ int attention_impl(yx_ctx* c, yx_kv* kv, size_t layer, const float* q, float* ou
     return fail(YX_ERR_INVALID, "internal: write_rows cannot be fused here");
   const float scale_log2 = scale * yx::kLog2e;
   dim3 grid(static_cast<unsigned>(plan->items.size()), static_cast<unsigned>(hkv));
+  const uint32_t by_item = plan->by_item ? 1u : 0u;
+  if (plan->by_item) grid = dim3(static_cast<unsigned>(hkv), static_cast<unsigned>(plan->items.size()));
   hipEvent_t e0;
   if ((rc = prof_begin(c, YX_KERNEL_ATTENTION, &e0))) return rc;
   const auto* items = static_cast<const yx::AttnItem*>(d_items);
@@ -1133,13 +1240,13 @@ int attention_impl(yx_ctx* c, yx_kv* kv, size_t layer, const float* q, float* ou
     hipLaunchKernelGGL(yx::paged_attn_decode_f32, grid, dim3(64 * yx::kWideWaves), 0, c->stream,
                        items, pos, pages, kv->kf(layer), kv->vf(layer), q, out, po, pml, cnt, knew,
                        vnew, c->dev_slot, kv->kf(layer),
-                       kv->vf(layer), po_bytes, pml_bytes, H, HK, P, W, scale_log2, mem);
+                       kv->vf(layer), po_bytes, pml_bytes, H, HK, P, W, scale_log2, mem, by_item);
   } else if (plan->balanced && !plan->wide) {
 #define YX_LAUNCH_BAL(QKV, UB, KN, VN, IN)                                                          \
   hipLaunchKernelGGL((yx::paged_attn_decode_balanced<QKV, UB>), grid, dim3(64 * yx::kBalWaves), 0,  \
                      c->stream, items, pos, pages, kv->k[layer], kv->v[layer], q, out, po, pml,     \
                      cnt, KN, VN, c->dev_slot, kv->k[layer],        \
-                     kv->v[layer], po_bytes, pml_bytes, H, HK, P, W, scale_log2, IN)
+                     kv->v[layer], po_bytes, pml_bytes, H, HK, P, W, scale_log2, IN, by_item)
     if (qkv && plan->small_units) YX_LAUNCH_BAL(true, 2, nullptr, nullptr, *qkv);
     else if (qkv) YX_LAUNCH_BAL(true, 4, nullptr, nullptr, *qkv);
     else if (plan->small_units) YX_LAUNCH_BAL(false, 2, knew, vnew, yx::QkvIn{});
@@ -1150,7 +1257,7 @@ int attention_impl(yx_ctx* c, yx_kv* kv, size_t layer, const float* q, float* ou
   hipLaunchKernelGGL((yx::paged_attn_decode_wide<NT, QKV, CASC>), grid, dim3(64 * yx::kWideWaves), 0, \
                      c->stream, items, pos, pages, kv->k[layer], kv->v[layer], q, out, po, pml,     \
                      cnt, KN, VN, c->dev_slot, kv->k[layer],        \
-                     kv->v[layer], po_bytes, pml_bytes, H, HK, P, W, scale_log2, IN, mem)
+                     kv->v[layer], po_bytes, pml_bytes, H, HK, P, W, scale_log2, IN, mem, by_item)
     const bool casc = plan->cascades > 0;  // shared prefixes only in one-tile passes
     if (qkv && casc) YX_LAUNCH_WIDE(1, true, nullptr, nullptr, *qkv, true);
     else if (qkv) YX_LAUNCH_WIDE(1, true, nullptr, nullptr, *qkv, false);
