@@ -43,3 +43,37 @@ def test_ragged_pass(hip, batch, rows, lo, hi, hq, hkv, page, window, f32):
     finally:
         hip.set_option("attn_max_chunk_blocks", 1 << 20)
         sc.kv.destroy()
+
+
+@pytest.mark.parametrize("chunks,priors,hq,hkv,window,f32", [
+    ([512], [6000], 24, 4, 0, False),       # tiles of 60 logical rows in several rounds of chunks
+    ([512], [3000], 24, 4, 1024, False),    # one round: two chunks per tile
+    ([200, 200], [900, 5200], 16, 4, 0, False),
+    ([256], [2900], 24, 4, 0, True),        # the f32 arena
+])
+def test_prefill_chunks_of_long_tiles(hip, chunks, priors, hq, hkv, window, f32):
+    """Prefill tiles split along keys where chunks of the average load would leave a second,
+    mostly empty round: against the oracle, the unsplit pass and call to call."""
+    sc = Scenario(hip, pages=sum(-(-(a + b) // 64) for a, b in zip(chunks, priors)) + 8, page=64, hkv=hkv,
+                  pool_seed=3, f32=f32)
+    try:
+        seqs = [sc.cache.new_seq() for _ in chunks]
+        sc.prefill(dict(zip(seqs, priors)))
+        pr = sc.run_pass(list(zip(seqs, chunks)))
+        sc.store(pr)
+        rows = len(pr.meta.pos)
+        q = sc.draw(rows * hq * D).reshape(rows, hq * D)
+        split0 = hip.stat("prefill_split_tiles")
+        got = hip.attend(sc.kv, 0, q, hq, window=window)
+        assert hip.stat("prefill_split_tiles") > split0
+        again = hip.attend(sc.kv, 0, q, hq, window=window)
+        assert np.array_equal(got.view(np.uint32), again.view(np.uint32))
+        hip.set_option("prefill_split", 0)
+        whole = hip.attend(sc.kv, 0, q, hq, window=window)
+        assert np.abs(got - whole).max() < 2e-5
+        some = np.r_[0:8, rows // 2 - 4:rows // 2 + 4, rows - 8:rows]  # the oracle on a part of the rows
+        want = sc.orc[0].attend(q[some], hq, pr.meta.pos[some], pr.meta.pt_off[some], pr.meta.pages, window=window)
+        assert close(got[some], want).all() and np.abs(got[some] - want).max() < 2e-5
+    finally:
+        hip.set_option("prefill_split", 1)
+        sc.kv.destroy()

@@ -600,27 +600,97 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
         w.chunk_nch = 1u << 16;
         plan.pitems.push_back(w);
       }
-    // Tiles longer than 1.5 times the average load of a workgroup slot (two per CU; a
-    // long context with few tiles: one sequence's chunk after thousands of keys) are
-    // split along keys into chunks of about that load, at least kMinChunkPairs pairs of
-    // blocks each; the chunks' partial results are merged by the tile's last chunk.
-    // (cfg3's tiles, 1024 over 512 slots, stay whole.)
+    // Tiles may be split along keys into chunks (at least kMinChunkPairs pairs of blocks
+    // each), merged by the tile's last chunk: a long context with few tiles, or a few
+    // tiles much longer than the others. The chunk length with the smallest estimated time
+    // among: none; about the average load of a workgroup slot for tiles over 1.5 times that;
+    // and fractions and multiples of it, since chunks of the average load give one and a
+    // bit rounds (208 tiles of 1516 pairs over 512 slots: 3 chunks each, 624 items in two
+    // rounds of 505 pairs; 12 chunks, five rounds of 126). The estimate deals the items,
+    // longest first, to the slots of one head (the heads' items are alike): an item's
+    // pairs plus kFixedPairs (its start and output) and, split, kSplitPairs (partial
+    // results and merge). In several rounds the part above the balance counts kTail, since
+    // a CU with one item left runs it faster; with at most one item per two slots every CU
+    // does, at 0.8 of the time per pair of two side by side. Splitting only where the plain choice is more than
+    // 1.08 times a perfect balance keeps the search off most passes. Measured (us per layer,
+    // write_rows included, chunks of the average load -> this): 512 rows after 24000 keys,
+    // 24/4 heads, full 444 -> 360, window 2048 63.6 -> 53.6; f32, 512 rows after 3000: 332
+    // -> 245; 2 x 483 rows after 904 and 11780, 16/4: 127 (128 with kSplitPairs 8, 133 with
+    // 3 and more chunks); kTail 1 picks as many chunks again.
     if (c->prefill_split) {
-      constexpr uint64_t kFixedPairs = 4;     // a tile's start and output, in pairs
-      constexpr uint32_t kMinChunkPairs = 16;
+      constexpr double kTail = 0.5;
+      constexpr uint32_t kFixedPairs = 7, kSplitPairs = 8, kMinChunkPairs = 16;
       uint64_t total = 0;
-      for (const yx::PrefillItem& w : plan.pitems) total += (w.blk1 - w.blk0 + 1) / 2 + kFixedPairs;
+      for (const yx::PrefillItem& w : plan.pitems) total += (w.blk1 - w.blk0 + 1) / 2 + 4;
       total *= hkv;
       // Workgroup slots: two per CU (4-wave tiles), one (8-wave f32 tiles).
-      const uint64_t slots2 = (f32 && plan.pf32_waves == 8 ? 1 : 2) * static_cast<uint64_t>(c->cus);
-      const uint64_t avg = std::max<uint64_t>(kMinChunkPairs, (total + slots2 - 1) / slots2);
+      const uint32_t per_cu = f32 && plan.pf32_waves == 8 ? 1 : 2;
+      const uint64_t slots2 = per_cu * static_cast<uint64_t>(c->cus);
+      const uint32_t avg = static_cast<uint32_t>(std::max<uint64_t>(kMinChunkPairs, (total + slots2 - 1) / slots2));
+      struct Split {
+        uint32_t pairs, over;  // chunks of about `pairs`, for tiles of more than `over` (0: none)
+      };
+      auto chunks = [&](uint32_t pairs, const Split& sp) {
+        if (!sp.pairs || pairs <= sp.over) return 1u;
+        return std::max(1u, std::min({(pairs + sp.pairs - 1) / sp.pairs, pairs / kMinChunkPairs, 64u}));
+      };
+      std::vector<uint32_t> lens, load;
+      size_t parts = 0;       // partial slots of the split last estimated
+      double balance = 0;     // and its load per slot
+      // At least `cutoff`: the balance alone says so (the deal is left out).
+      auto estimate = [&](const Split& sp, double cutoff) {
+        lens.clear();
+        parts = 0;
+        uint64_t sum = 0;
+        for (const yx::PrefillItem& w : plan.pitems) {
+          const uint32_t pairs = (w.blk1 - w.blk0 + 1) / 2, nch = chunks(pairs, sp);
+          if (nch > 1) parts += nch;
+          for (uint32_t ch = 0; ch < nch; ++ch) {
+            const uint32_t n = static_cast<uint32_t>(static_cast<uint64_t>(pairs) * (ch + 1) / nch) -
+                               static_cast<uint32_t>(static_cast<uint64_t>(pairs) * ch / nch);
+            lens.push_back(n + kFixedPairs + (nch > 1 ? kSplitPairs : 0));
+            sum += lens.back();
+          }
+        }
+        load.assign(std::max<size_t>(1, slots2 / hkv), 0);
+        balance = static_cast<double>(sum) / load.size();
+        if (balance >= cutoff) return balance;
+        std::sort(lens.begin(), lens.end(), std::greater<uint32_t>());
+        uint32_t most = 0;
+        for (uint32_t n : lens) {  // a min-heap of the slots' loads
+          std::pop_heap(load.begin(), load.end(), std::greater<uint32_t>());
+          load.back() += n;
+          most = std::max(most, load.back());
+          std::push_heap(load.begin(), load.end(), std::greater<uint32_t>());
+        }
+        if (lens.size() > load.size()) return balance + kTail * (most - balance);
+        return (per_cu == 2 && lens.size() * 2 <= load.size() ? 0.8 : 1.0) * most;
+      };
+      // Partials that fit the scratch of the entry point that allocates nothing keep fitting.
+      const size_t part_bytes = hkv * tile_rows * (yx::kD * sizeof(float) + sizeof(float2));
+      const size_t scratch = kScratchBytes - kScratchCounterBytes - kScratchListBytes - 4096;
+      Split best{avg, avg + avg / 2};
+      double best_t = estimate(best, 1e30);
+      const size_t plain_parts = parts;
+      if (best_t > 1.08 * balance) {
+        auto consider = [&](const Split& sp) {
+          const double t = estimate(sp, 0.98 * best_t);
+          if (t < 0.98 * best_t && (parts * part_bytes <= scratch || plain_parts * part_bytes > scratch) &&
+              parts * part_bytes <= (size_t{1} << 30)) {
+            best = sp;
+            best_t = t;
+          }
+        };
+        consider(Split{0, 0});
+        for (uint32_t pc : {20, 28, 40, 56, 80, 120, 180}) {
+          const uint32_t n = std::max(kMinChunkPairs, avg * pc / 100);
+          consider(Split{n, n});
+        }
+      }
       std::vector<yx::PrefillItem> split;
       uint32_t nslot = 0, ncnt = 0;
       for (const yx::PrefillItem& w : plan.pitems) {
-        const uint32_t pairs = (w.blk1 - w.blk0 + 1) / 2;
-        uint32_t nch = 1;
-        if (2 * static_cast<uint64_t>(pairs) > 3 * avg)
-          nch = static_cast<uint32_t>(std::min<uint64_t>({(pairs + avg - 1) / avg, pairs / kMinChunkPairs, 64}));
+        const uint32_t pairs = (w.blk1 - w.blk0 + 1) / 2, nch = chunks(pairs, best);
         if (nch <= 1) {
           split.push_back(w);
           continue;
@@ -820,8 +890,8 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
   // 38.2 -> 29.6; 30 of 2000-2100, 16/4: 38.4 -> 28.1; 5 of 16000-20000, 16/8: 84.2 ->
   // 63.5; verify, 20 x 4 rows after 200-6000: 31.9 -> 22.2; f32, 20 of 200-9000, 16/8:
   // 102.8 -> 78.8.
-  std::vector<uint32_t> lens;
-  auto estimate = [&](size_t cbk) {
+  std::vector<uint32_t> lens, load;
+  auto estimate = [&](size_t cbk, double cutoff) {
     constexpr uint32_t kStartBlocks = 16;
     constexpr double kTail = 0.6;
     lens.clear();
@@ -832,19 +902,20 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
     };
     for (const Casc& cc : cascs) add(cc.blocks);
     for (const Sub& sb : subs) add(sb.b1 - sb.b0);
-    std::sort(lens.begin(), lens.end(), std::greater<uint32_t>());
     // Slots of one head: the heads' items are alike.
-    std::vector<uint32_t> load(std::max<size_t>(1, static_cast<size_t>(c->cus) / hkv), 0);
+    load.assign(std::max<size_t>(1, static_cast<size_t>(c->cus) / hkv), 0);
     uint64_t total = 0;
+    for (uint32_t n : lens) total += n;
+    const double avg = static_cast<double>(total) / load.size();
+    if (avg >= cutoff) return avg;  // no deal is better than the average
+    std::sort(lens.begin(), lens.end(), std::greater<uint32_t>());
     uint32_t most = 0;
     for (uint32_t n : lens) {  // min-heap of the slots' loads
       std::pop_heap(load.begin(), load.end(), std::greater<uint32_t>());
       load.back() += n;
       most = std::max(most, load.back());
       std::push_heap(load.begin(), load.end(), std::greater<uint32_t>());
-      total += n;
     }
-    const double avg = static_cast<double>(total) / load.size();
     return avg + kTail * (most - avg);
   };
   bool sort_items = false;
@@ -874,12 +945,12 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
       const size_t items0 = items_of(cb, &slots0);
       const size_t max_slots = std::max<size_t>(slots0, 640), max_items = std::max<size_t>(items0, 8192);
       size_t best = cb;
-      double best_t = estimate(cb);
+      double best_t = estimate(cb, 1e30);
       auto consider = [&](size_t cbk) {
         cbk = std::min(std::max<size_t>(cbk, 16), limit);
         size_t sl;
         if (items_of(cbk, &sl) > max_items || sl > max_slots) return;
-        const double t = estimate(cbk);
+        const double t = estimate(cbk, best_t);
         if (t < best_t) {
           best_t = t;
           best = cbk;
