@@ -77,8 +77,8 @@ int yx_sync(yx_ctx* ctx);
  * tile along k, at most 64; 0, the default: automatic; it changes the result only by
  * the order of the f32 additions), "argmax_slices" (workgroups per yx_argmax_rows_dev
  * row, at most 1024; 0, the default: automatic; the result does not change) and
- * "prefill_f32_waves" (the f32 arena's prefill tiles: 8 waves of 16 logical rows or 4;
- * 0, the default: 4 when every sequence of the pass has at most 64 logical rows). Setting an
+ * "prefill_f32_waves" (the f32 arena's prefill tiles: 8 waves of 16 logical rows, on
+ * products of bf16 parts, or 4, on f32 products; 0, the default: 8). Setting an
  * option drops cached work lists. Values are positive; 0 is accepted for
  * attn_target_waves, attn_decode_shape, attn_cascade, attn_xcd_prefix, prefill_split, prefill_min_rows,
  * matmul_k_split, argmax_slices and prefill_f32_waves (which takes 0, 4 or 8). */
@@ -94,8 +94,9 @@ int yx_ctx_get_stat(yx_ctx* ctx, const char* key, uint64_t* out);
 /* Backend::new_kv (lib.rs:118; GPU ops/mod.rs:42-66): `layers` layers of `pages`
  * pages of `page_size` tokens (a multiple of 16), zeroed. dtype YX_DTYPE_F16 (binary16,
  * the fast path) or YX_DTYPE_F32 (the reference's own K/V precision: stores are exact,
- * attention runs on f32 MFMAs: split-K decode items of at most 16 (row, q head) pairs,
- * or prefill tiles of 128 or 64, chosen as the options prefill_min_rows and
+ * attention at f32's precision: split-K decode items of at most 16 (row, q head) pairs on
+ * f32 MFMAs, or prefill tiles of 128 or 64 (the 128 on exact bf16 parts of the f32 values,
+ * except where those would not do), chosen as the options prefill_min_rows and
  * prefill_f32_waves of yx_ctx_set_option describe;
  * at most 16 q heads per KV head; write_rows as its own launch). */
 int yx_kv_create(yx_ctx* ctx, size_t layers, size_t pages, size_t page_size, size_t hkv,

@@ -1,0 +1,94 @@
+"""The f32 arena's prefill tiles of 128 logical rows, which multiply bf16 parts of the f32
+values, against the tiles of 64 (f32 products): ordinary values, magnitudes that parts
+still serve, and those handed over to f32 products (infinities, large K or q, small V)."""
+
+import numpy as np
+import pytest
+
+from tests.scenario import D, Scenario
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("ks,qs,vs,scale,bad,window", [
+    (1.0, 1.0, 1.0, None, None, 0),
+    (1.0, 1.0, 1.0, None, None, 129),
+    (1.0, 1.0, 1.0, -0.11, None, 0),          # the smallest score leads
+    (1.0, 1.0, 1.0, 0.0, None, 0),            # equal weights
+    (2.0**60, 2.0**-60, 2.0**100, None, None, 0),
+    (2.0**-60, 2.0**60, 2.0**-80, None, None, 0),
+    (2.0**100, 2.0**-100, 1.0, None, None, 0),   # K above what parts serve
+    (2.0**-100, 2.0**100, 1.0, None, None, 33),  # q above
+    (2.0**-100, 2.0**-10, 1.0, 2.0**107, None, 0),  # the scale above
+    (1.0, 1.0, 2.0**-120, None, None, 0),        # V below
+    (1.0, 1.0, 1.0, None, ("k", np.inf), 0),
+    (1.0, 1.0, 1.0, None, ("v", -np.inf), 40),
+    (1.0, 1.0, 1.0, None, ("v", np.nan), 40),
+    (1.0, 1.0, 2.0**105, None, None, 0),
+])
+def test_parts_match_f32_products(hip, ks, qs, vs, scale, bad, window):
+    hq, hkv, rows = 8, 2, [1000, 37, 1]  # split tiles, a ragged tile, one row
+    sc = Scenario(hip, pages=sum(-(-r // 32) for r in rows) + 4, page=32, hkv=hkv, pool_seed=5, f32=True)
+    try:
+        seqs = [sc.cache.new_seq() for _ in rows]
+        pr = sc.run_pass(list(zip(seqs, rows)))
+        t = len(pr.meta.pos)
+        k, v = (sc.draw(t * hkv * D).reshape(t, hkv, D) for _ in range(2))
+        q = sc.draw(t * hq * D).reshape(t, hq * D) * np.float32(qs)
+        k = k * np.float32(ks)
+        v = v / np.abs(v).max() * np.float32(vs)
+        if bad:
+            {"k": k, "v": v}[bad[0]][500, 1, 77] = bad[1]
+        hip.set_option("prefill_min_rows", 1)
+        # Whole tiles with an infinity: a merge skips a chunk whose sum is NaN, and the two
+        # shapes cut their tiles in different places.
+        hip.set_option("prefill_split", int(not bad))
+        out = {}
+        for waves in (8, 4):
+            hip.set_option("prefill_f32_waves", waves)
+            split0 = hip.stat("prefill_split_tiles")
+            out[waves] = hip.attend_append(sc.kv, 0, k, v, q, hq, window=window, scale=scale)
+            assert hip.stat("prefill_split_tiles") > split0 or window or bad
+        a, b = (np.asarray(x, np.float64) for x in (out[8], out[4]))
+        assert np.array_equal(np.isnan(a), np.isnan(b))
+        assert np.array_equal(np.isinf(a), np.isinf(b))
+        assert (bad is not None) == bool((~np.isfinite(b)).any())
+        # A score's rounding (128 products of unit size) and an output's, each a few 2^-24 of
+        # the largest value, on either side.
+        ok = np.isfinite(a)
+        assert np.abs(a[ok] - b[ok]).max() < 4e-6 * vs
+        assert np.linalg.norm(a[ok] / vs - b[ok] / vs) < 2e-6 * np.linalg.norm(b[ok] / vs)
+    finally:
+        hip.set_option("prefill_min_rows", 0)
+        hip.set_option("prefill_f32_waves", 0)
+        hip.set_option("prefill_split", 1)
+        sc.kv.destroy()
+
+
+@pytest.mark.parametrize("rows,prior,hq,hkv", [
+    (8, 4096, 16, 4),    # tiles with a quarter of their rows, partial slots of 32
+    (5, 1500, 12, 4),    # 15 logical rows: stays decode items
+    (11, 2000, 12, 4),   # 33
+])
+def test_few_rows_per_tile(hip, rows, prior, hq, hkv):
+    """Passes with few rows after a long context (partial slots of the rows in use): the
+    automatic choice, decode items and tiles against the oracle's f64 form."""
+    sc = Scenario(hip, pages=4 * (-(-(rows + prior) // 64)) + 4, page=64, hkv=hkv, pool_seed=9, f32=True)
+    try:
+        seqs = [sc.cache.new_seq() for _ in range(4)]
+        sc.prefill({s: prior - 7 * i for i, s in enumerate(seqs)})
+        pr = sc.run_pass([(s, rows) for s in seqs])
+        sc.store(pr)
+        t = len(pr.meta.pos)
+        q = sc.draw(t * hq * D).reshape(t, hq * D)
+        auto = hip.attend(sc.kv, 0, q, hq)
+        hip.set_option("prefill_min_rows", 1 << 20)
+        items = hip.attend(sc.kv, 0, q, hq)
+        hip.set_option("prefill_min_rows", 1)
+        tiles = hip.attend(sc.kv, 0, q, hq)
+        want = sc.orc[0].attend_f64(q, hq, pr.meta.pos, pr.meta.pt_off, pr.meta.pages)
+        for x in (auto, items, tiles):
+            assert np.abs(x - want).max() < 1e-5
+    finally:
+        hip.set_option("prefill_min_rows", 0)
+        sc.kv.destroy()

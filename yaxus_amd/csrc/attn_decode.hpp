@@ -160,6 +160,13 @@ __device__ __forceinline__ void load_block(BlockRegs& r, const _Float16* __restr
   for (int i = 0; i < 4; ++i) r.v[i] = __builtin_nontemporal_load(vp + i * (kD / 8));
 }
 
+// A workgroup barrier that orders LDS accesses only: global loads stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Waves per workgroup (W): they share one work item's blocks and merge through LDS.
 // With one tile a wave needs ~220 registers, so eight waves (two per SIMD) fit a CU and
 // keep twice the loads in flight that four do; more tiles need more than 256 registers

@@ -60,12 +60,13 @@ struct PrefillItem {
 // sum, unnormalised O) of each logical row in chunk slots base .. base + nch - 1, in
 // chunk order, so the result does not depend on arrival order. A thread takes kPer
 // (row, 4 dims) entries, kGE at a time, and has the loads of kCB chunks of those kGE
-// entries in flight at once (a tile's partials are many: 64 or 128 rows per chunk).
+// entries in flight at once (a tile's partials are many: 64 or 128 rows per chunk). A
+// partial slot holds part_rows rows.
 template <int kThreads, int kRows>
 __device__ __forceinline__ void merge_tile(uint32_t r0, uint32_t nrows, uint32_t base, uint32_t nch,
                                            uint32_t kh, uint32_t G, uint32_t hq, uint32_t hkv,
                                            float* __restrict__ out, __amdgpu_buffer_rsrc_t ro,
-                                           __amdgpu_buffer_rsrc_t rml) {
+                                           __amdgpu_buffer_rsrc_t rml, uint32_t part_rows = kRows) {
   constexpr int kPer = kRows * 32 / kThreads;
   constexpr int kGE = 4, kCB = 4;
   static_assert(kPer % kGE == 0, "whole groups of entries per thread");
@@ -93,7 +94,7 @@ __device__ __forceinline__ void merge_tile(uint32_t r0, uint32_t nrows, uint32_t
 #pragma unroll
         for (int b = 0; b < kCB; ++b) {
           const uint32_t ch = min(c0 + b, nch - 1);
-          const size_t e = ((static_cast<size_t>(base) + ch) * hkv + kh) * kRows + (lr[j] < nlog ? lr[j] : 0u);
+          const size_t e = ((static_cast<size_t>(base) + ch) * hkv + kh) * part_rows + (lr[j] < nlog ? lr[j] : 0u);
           ml[j][b] = ld2_coherent(rml, static_cast<uint32_t>(e * 8));
           po[j][b] = ld4_coherent(ro, static_cast<uint32_t>((e * kD + qi[j] * 4) * 4));
         }

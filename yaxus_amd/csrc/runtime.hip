@@ -180,6 +180,7 @@ struct AttnPlan {
   bool fusable = false;  // the append can run inside the attention kernel
   bool by_item = false;  // decode grid (hkv, items): items in list order, all heads of each in turn
   size_t slots = 0;     // partial slots (per kv head)
+  uint32_t part_rows = 0;  // logical rows of a partial slot (prefill)
   size_t counters = 0;  // arrival counters (per kv head)
   bool uploaded = false;  // dev_items / dev_members hold the lists
   // Where the kernels read the lists: d_items / d_members, or the pass's metadata buffer
@@ -530,22 +531,22 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
   // ctx, decode / prefill us): 16 x 10 after 4096 57.1 / 49.5, 16 x 8 34.2 / 43.0, 1 x 32
   // after 32768 50.1 / 101.1, 1 x 128 after 32768 218.1 / 103.6, 2 x 64 after 16384
   // 81.5 / 70.7.
-  bool use_prefill;
+  bool use_prefill, must_fit = false;
   if (c->prefill_min_rows > 0) {
     use_prefill = max_rows >= static_cast<uint32_t>(c->prefill_min_rows);
   } else if (f32) {
     // The f32 arena: its decode items hold 16 logical rows each and re-read their
-    // sequence's keys once per item (about 6 TB/s over those reads); its prefill tiles
-    // (64 or 128 logical rows, 8 waves per CU) take about 95 us plus 2.4 us per 1024 keys
-    // of the longest context (the key split's chain), or 40 us plus their products at
-    // 110 TFLOP/s, whichever is more. The kernel with the smaller estimate runs. Measured
-    // (B x rows after ctx, decode / prefill us; the choice was right in 19 of 21 shapes,
-    // the two misses 5% and 30%): 1 x 32 after 4096 32.6 / 101.8, 1 x 128 after 4096
-    // 83.9 / 107.2, 32 x 8 after 2048 94.8 / 119.2, 1 x 48 after 16384 186.6 / 133.4,
-    // 1 x 96 after 8192 197.4 / 118.9, 4 x 32 after 8192 177.6 / 129.5, 16 x 10 after
-    // 4096 172.0 / 127.6, 1 x 32 after 32768 137.7 / 178.7, 1 x 64 after 32768
-    // 453.3 / 217.3, 16 x 256 after 1024 812.5 / 352.8.
-    double decode_bytes = 0, flops = 0;
+    // sequence's keys once per item (about 6 TB/s over those reads). A prefill tile (one
+    // workgroup, 128 logical rows) takes 2.0 us per 32 keys, 2.9 with all its rows in use;
+    // the pass takes the busiest CU's share, but no tile is cut below about 11 such stages,
+    // and a cut tile's merge 1.2 us per chunk. The kernel with the smaller estimate runs.
+    // Measured (B x rows after ctx, 16/4 heads, decode / prefill us with the append):
+    // 1 x 64 after 4096 43.9 / 57.8, 1 x 128 78.6 / 65.6, 1 x 256 158 / 71.6, 4 x 64 after
+    // 1024 54.7 / 44.3, 16 x 8 after 4096 98.3 / 80.7, 16 x 10 158 / 92.9, 32 x 16 after 512
+    // 56.2 / 44.4, 1 x 32 after 16384 69.1 / 94.6, 1 x 48 139 / 94.9, 1 x 32 after 32768
+    // 125 / 128, 1 x 64 445 / 141, 16 x 256 after 1024 745 / 227; the choice was right in 53
+    // of 56 shapes (16/4 and 16/8 heads), the misses 5, 8 and 16%.
+    double decode_bytes = 0, stages = 0, used = 0, tiles = 0;
     uint32_t max_keys = 0;
     for (const Group& g : c->groups) {
       uint32_t keys = 0;
@@ -553,13 +554,23 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
       if (window > 0) keys = static_cast<uint32_t>(std::min<uint64_t>(keys, window + g.n));
       max_keys = std::max(max_keys, keys);
       decode_bytes += static_cast<double>((g.n * G + 15) / 16) * keys;
-      flops += static_cast<double>(g.n) * G * keys;
+      const double t = static_cast<double>((g.n * G + yx::kPf32Rows - 1) / yx::kPf32Rows);
+      tiles += t;
+      stages += t * keys / 32;
+      used += static_cast<double>(g.n) * G / yx::kPf32Rows * keys / 32;
     }
     decode_bytes *= static_cast<double>(hkv) * yx::kD * sizeof(float) * 2;
-    flops *= static_cast<double>(hkv) * 4 * yx::kD;
     const double decode_us = decode_bytes / 6e6;
-    const double prefill_us = std::max(95.0 + 2.4 * max_keys / 1024.0, 40.0 + flops / 1.1e8);
+    constexpr double kShort = 11;
+    const double longest = max_keys / 32.0;
+    const double share = std::max(stages * hkv / c->cus, std::min(kShort, longest));
+    const double cuts = std::min({64.0, c->cus / (tiles * hkv), longest / kShort});
+    const double prefill_us = 10 + share * (2.0 + 0.9 * used / stages) + (cuts > 1 ? 1.2 * cuts : 0);
     use_prefill = max_rows * G > 16 && decode_us > prefill_us;
+    // Decode items serve a pass this short through the entry point that allocates nothing:
+    // tiles take it only if their partials fit that scratch too (not, for one, those of
+    // 4 x 64 chunks of 128 rows after 28000 keys).
+    must_fit = decode_us <= 95.0 + 2.4 * max_keys / 1024.0;
   } else {
     size_t tiles = 0;
     for (const Group& g : c->groups) tiles += (g.n * G + yx::kPrefillRows - 1) / yx::kPrefillRows;
@@ -568,19 +579,17 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
                   tiles * 8 >= static_cast<size_t>(c->cus);
   }
   if (use_prefill) {
-    ++c->prefill_plans;
     // Tiles of kPrefillRows logical rows: consecutive rows of one sequence (the f16 and
     // the f32 arena's prefill kernels take the same items).
     AttnPlan plan;
     plan.prefill = true;
     plan.f32 = f32;
-    // f32 tiles of 64 logical rows (two 4-wave workgroups per CU) when every sequence's
-    // rows fit one (option prefill_f32_waves: 4 or 8 fixes the shape).
-    if (f32)
-      plan.pf32_waves = c->pf32_waves ? static_cast<int>(c->pf32_waves)
-                                      : (max_rows * G <= static_cast<size_t>(yx::kPf32SmallRows) ? 4 : 8);
+    // f32 tiles of 128 logical rows (option prefill_f32_waves: 4 takes 64, on f32 products).
+    if (f32) plan.pf32_waves = c->pf32_waves ? static_cast<int>(c->pf32_waves) : 8;
     const size_t tile_rows = !f32 ? yx::kPrefillRows : plan.pf32_waves == 4 ? yx::kPf32SmallRows : yx::kPf32Rows;
     const uint32_t per = static_cast<uint32_t>(std::max<size_t>(1, tile_rows / G));
+    // f32 partials hold the rows in use (a tile of few rows and many chunks).
+    plan.part_rows = static_cast<uint32_t>(!f32 ? tile_rows : std::min<size_t>(tile_rows, max_rows * G));
     if (G > tile_rows)
       return fail(YX_ERR_UNSUPPORTED, "more query heads per KV head than a prefill tile holds");
     for (const Group& g : c->groups)
@@ -611,15 +620,24 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
     // pairs plus kFixedPairs (its start and output) and, split, kSplitPairs (partial
     // results and merge). In several rounds the part above the balance counts kTail, since
     // a CU with one item left runs it faster; with at most one item per two slots every CU
-    // does, at 0.8 of the time per pair of two side by side. Splitting only where the plain choice is more than
-    // 1.08 times a perfect balance keeps the search off most passes. Measured (us per layer,
+    // does, at 0.8 of the time per pair of two side by side. Splitting only where the plain
+    // choice is more than 1.08 times a perfect balance keeps the search off most passes. f32
+    // tiles on parts take 2.9 us per pair, so their fixed costs are fewer pairs, chunks down
+    // to 8 pairs pay (8 against 16: 4 x 64 rows after 1024 keys 64 -> 44, 1 x 128 after 512
+    // 62 -> 45, 1 x 64 after 4096 69 -> 58) and the merge counts, nch / 3 pairs (32 chunks
+    // against 64: 1 x 32 after 16384 94 / 103). Measured (us per layer,
     // write_rows included, chunks of the average load -> this): 512 rows after 24000 keys,
     // 24/4 heads, full 444 -> 360, window 2048 63.6 -> 53.6; f32, 512 rows after 3000: 332
     // -> 245; 2 x 483 rows after 904 and 11780, 16/4: 127 (128 with kSplitPairs 8, 133 with
     // 3 and more chunks); kTail 1 picks as many chunks again.
     if (c->prefill_split) {
       constexpr double kTail = 0.5;
-      constexpr uint32_t kFixedPairs = 7, kSplitPairs = 8, kMinChunkPairs = 16;
+      constexpr uint32_t kMinChunkPairs = 16;
+      const bool parts8 = f32 && plan.pf32_waves == 8;
+      const uint32_t kFixedPairs = parts8 ? 3 : 7, kSplitPairs = parts8 ? 4 : 8;
+      const uint32_t min_chunk = parts8 ? 8 : kMinChunkPairs;
+      // A chunk's own cost in a tile of nch, in pairs.
+      auto split_cost = [&](uint32_t nch) { return nch <= 1 ? 0 : kSplitPairs + (parts8 ? nch / 3 : 0); };
       uint64_t total = 0;
       for (const yx::PrefillItem& w : plan.pitems) total += (w.blk1 - w.blk0 + 1) / 2 + 4;
       total *= hkv;
@@ -632,7 +650,7 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
       };
       auto chunks = [&](uint32_t pairs, const Split& sp) {
         if (!sp.pairs || pairs <= sp.over) return 1u;
-        return std::max(1u, std::min({(pairs + sp.pairs - 1) / sp.pairs, pairs / kMinChunkPairs, 64u}));
+        return std::max(1u, std::min({(pairs + sp.pairs - 1) / sp.pairs, pairs / std::min(sp.pairs, kMinChunkPairs), 64u}));
       };
       std::vector<uint32_t> lens, load;
       size_t parts = 0;       // partial slots of the split last estimated
@@ -648,7 +666,7 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
           for (uint32_t ch = 0; ch < nch; ++ch) {
             const uint32_t n = static_cast<uint32_t>(static_cast<uint64_t>(pairs) * (ch + 1) / nch) -
                                static_cast<uint32_t>(static_cast<uint64_t>(pairs) * ch / nch);
-            lens.push_back(n + kFixedPairs + (nch > 1 ? kSplitPairs : 0));
+            lens.push_back(n + kFixedPairs + split_cost(nch));
             sum += lens.back();
           }
         }
@@ -667,11 +685,12 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
         return (per_cu == 2 && lens.size() * 2 <= load.size() ? 0.8 : 1.0) * most;
       };
       // Partials that fit the scratch of the entry point that allocates nothing keep fitting.
-      const size_t part_bytes = hkv * tile_rows * (yx::kD * sizeof(float) + sizeof(float2));
+      const size_t part_bytes = hkv * plan.part_rows * (yx::kD * sizeof(float) + sizeof(float2));
       const size_t scratch = kScratchBytes - kScratchCounterBytes - kScratchListBytes - 4096;
       Split best{avg, avg + avg / 2};
       double best_t = estimate(best, 1e30);
       const size_t plain_parts = parts;
+      size_t chosen_parts = parts;
       if (best_t > 1.08 * balance) {
         auto consider = [&](const Split& sp) {
           const double t = estimate(sp, 0.98 * best_t);
@@ -679,14 +698,16 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
               parts * part_bytes <= (size_t{1} << 30)) {
             best = sp;
             best_t = t;
+            chosen_parts = parts;
           }
         };
         consider(Split{0, 0});
         for (uint32_t pc : {20, 28, 40, 56, 80, 120, 180}) {
-          const uint32_t n = std::max(kMinChunkPairs, avg * pc / 100);
+          const uint32_t n = std::max(min_chunk, avg * pc / 100);
           consider(Split{n, n});
         }
       }
+      if (must_fit && chosen_parts * part_bytes > scratch) use_prefill = false;
       std::vector<yx::PrefillItem> split;
       uint32_t nslot = 0, ncnt = 0;
       for (const yx::PrefillItem& w : plan.pitems) {
@@ -711,18 +732,21 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
       plan.pitems = std::move(split);
       plan.slots = nslot;
       plan.counters = ncnt;
-      c->split_tiles += ncnt;
+      if (use_prefill) c->split_tiles += ncnt;
     }
-    // Longest first: the GPU hands work items to CUs in order as they free up, so
-    // this bounds the busiest CU near the average (contexts differ a lot in a pass).
-    std::stable_sort(plan.pitems.begin(), plan.pitems.end(),
-                     [](const yx::PrefillItem& a, const yx::PrefillItem& b) {
-                       return a.blk1 - a.blk0 > b.blk1 - b.blk0;
-                     });
-    auto& p = c->plans[key];
-    p = std::move(plan);
-    *out = &p;
-    return YX_OK;
+    if (use_prefill) {
+      ++c->prefill_plans;
+      // Longest first: the GPU hands work items to CUs in order as they free up, so
+      // this bounds the busiest CU near the average (contexts differ a lot in a pass).
+      std::stable_sort(plan.pitems.begin(), plan.pitems.end(),
+                       [](const yx::PrefillItem& a, const yx::PrefillItem& b) {
+                         return a.blk1 - a.blk0 > b.blk1 - b.blk0;
+                       });
+      auto& p = c->plans[key];
+      p = std::move(plan);
+      *out = &p;
+      return YX_OK;
+    }
   }
   size_t nt = (max_rows * G + 7) / 8;
   const long cap = f32 ? 2 : c->decode_shape != 1 ? c->max_tiles : std::min<long>(c->max_tiles, 3);
@@ -1192,9 +1216,7 @@ int attention_impl(yx_ctx* c, yx_kv* kv, size_t layer, const float* q, float* ou
       c->used_keys.push_back(key);
   }
   // Logical rows per partial slot: the kernel's tile rows.
-  const size_t rps = plan->prefill ? static_cast<size_t>(!plan->f32 ? yx::kPrefillRows
-                                                       : plan->pf32_waves == 4 ? yx::kPf32SmallRows
-                                                                               : yx::kPf32Rows)
+  const size_t rps = plan->prefill ? plan->part_rows
                     : plan->wide    ? static_cast<size_t>((plan->nt + 1) / 2) * 16
                                     : static_cast<size_t>(plan->nt) * 8;
   const size_t po_need = plan->slots * hkv * rps * 128 * 4, pml_need = plan->slots * hkv * rps * 8;
@@ -1263,7 +1285,7 @@ int attention_impl(yx_ctx* c, yx_kv* kv, size_t layer, const float* q, float* ou
                          reinterpret_cast<const float*>(kv->v[layer]), q, out,
                          static_cast<uint32_t>(hq), static_cast<uint32_t>(hkv), shift,
                          static_cast<uint32_t>(window), scale * yx::kLog2e, po, pml, cnt,
-                         pf_po_bytes, pf_pml_bytes);
+                         pf_po_bytes, pf_pml_bytes, plan->part_rows);
     } else if (qkv)
       hipLaunchKernelGGL((yx::paged_attn_prefill<true>), pgrid, dim3(64 * yx::kPrefillWaves), 0, c->stream,
                        static_cast<const yx::PrefillItem*>(d_items),
