@@ -619,22 +619,24 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
     // longest first, to the slots of one head (the heads' items are alike): an item's
     // pairs plus kFixedPairs (its start and output) and, split, kSplitPairs (partial
     // results and merge). In several rounds the part above the balance counts kTail, since
-    // a CU with one item left runs it faster; with at most one item per two slots every CU
-    // does, at 0.8 of the time per pair of two side by side. Splitting only where the plain
+    // a CU with one item left runs it faster; in one round of two items side by side, what
+    // the longer of a CU's two has left counts kAlone. Splitting only where the plain
     // choice is more than 1.08 times a perfect balance keeps the search off most passes. f32
     // tiles on parts take 2.9 us per pair, so their fixed costs are fewer pairs, chunks down
     // to 8 pairs pay (8 against 16: 4 x 64 rows after 1024 keys 64 -> 44, 1 x 128 after 512
     // 62 -> 45, 1 x 64 after 4096 69 -> 58) and the merge counts, nch / 3 pairs (32 chunks
     // against 64: 1 x 32 after 16384 94 / 103). Measured (us per layer,
     // write_rows included, chunks of the average load -> this): 512 rows after 24000 keys,
-    // 24/4 heads, full 444 -> 360, window 2048 63.6 -> 53.6; f32, 512 rows after 3000: 332
-    // -> 245; 2 x 483 rows after 904 and 11780, 16/4: 127 (128 with kSplitPairs 8, 133 with
-    // 3 and more chunks); kTail 1 picks as many chunks again.
+    // 24/4 heads, full 444 -> 360, window 2048 63.6 -> 53.6; 3 x 243 after 764-2082, 16/4,
+    // 46 -> 36; 2 x 483 rows after 904 and 11780, 16/4: 127 (129 with kSplitPairs 12, 133
+    // with 3 and more chunks). With kSplitPairs 8 and kAlone 0.8, 7 x 281 after 934-1796
+    // split in vain (72 -> 81) and so did 2 x 277 after 344-5912 (9% slower); kTail 1 picks
+    // as many chunks again.
     if (c->prefill_split) {
-      constexpr double kTail = 0.5;
+      constexpr double kTail = 0.5, kAlone = 0.9;
       constexpr uint32_t kMinChunkPairs = 16;
       const bool parts8 = f32 && plan.pf32_waves == 8;
-      const uint32_t kFixedPairs = parts8 ? 3 : 7, kSplitPairs = parts8 ? 4 : 8;
+      const uint32_t kFixedPairs = parts8 ? 3 : 7, kSplitPairs = parts8 ? 4 : 12;
       const uint32_t min_chunk = parts8 ? 8 : kMinChunkPairs;
       // A chunk's own cost in a tile of nch, in pairs.
       auto split_cost = [&](uint32_t nch) { return nch <= 1 ? 0 : kSplitPairs + (parts8 ? nch / 3 : 0); };
@@ -674,6 +676,15 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
         balance = static_cast<double>(sum) / load.size();
         if (balance >= cutoff) return balance;
         std::sort(lens.begin(), lens.end(), std::greater<uint32_t>());
+        if (per_cu == 2 && lens.size() <= load.size()) {
+          const size_t cus = std::max<size_t>(1, load.size() / 2);
+          double most = 0;
+          for (size_t j = 0; j < std::min(cus, lens.size()); ++j) {
+            const double beside = j + cus < lens.size() ? lens[j + cus] : 0;
+            most = std::max(most, beside + kAlone * (lens[j] - beside));
+          }
+          return most;
+        }
         uint32_t most = 0;
         for (uint32_t n : lens) {  // a min-heap of the slots' loads
           std::pop_heap(load.begin(), load.end(), std::greater<uint32_t>());
@@ -681,8 +692,7 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
           most = std::max(most, load.back());
           std::push_heap(load.begin(), load.end(), std::greater<uint32_t>());
         }
-        if (lens.size() > load.size()) return balance + kTail * (most - balance);
-        return (per_cu == 2 && lens.size() * 2 <= load.size() ? 0.8 : 1.0) * most;
+        return lens.size() > load.size() ? balance + kTail * (most - balance) : most;
       };
       // Partials that fit the scratch of the entry point that allocates nothing keep fitting.
       const size_t part_bytes = hkv * plan.part_rows * (yx::kD * sizeof(float) + sizeof(float2));
