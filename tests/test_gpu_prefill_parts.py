@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from tests.scenario import D, Scenario
+from yaxus_amd._lib import check_hip
 
 pytestmark = pytest.mark.gpu
 
@@ -91,4 +92,36 @@ def test_few_rows_per_tile(hip, rows, prior, hq, hkv):
             assert np.abs(x - want).max() < 1e-5
     finally:
         hip.set_option("prefill_min_rows", 0)
+        sc.kv.destroy()
+
+
+@pytest.mark.parametrize("batch,rows,prior", [
+    (16, 8, 4096),    # tiles of 32 logical rows: 256 partial slots, more than whole tiles' scratch
+    (1, 32, 28000),   # tiles whose partials don't fit: decode items
+])
+def test_no_alloc_entry_takes_them(hip, batch, rows, prior):
+    """Passes that decode items serve within the fixed scratch keep being served there."""
+    hq, hkv = 16, 4
+    sc = Scenario(hip, pages=batch * -(-(rows + prior) // 128) + 4, page=128, hkv=hkv, pool_seed=2, f32=True)
+    tensors = []
+    try:
+        seqs = [sc.cache.new_seq() for _ in range(batch)]
+        sc.prefill({s: prior for s in seqs}, chunk=8192)
+        pr = sc.run_pass([(s, rows) for s in seqs])
+        t = len(pr.meta.pos)
+        for n in (hkv, hkv, hq):
+            tensors.append(hip.tensor((t, n * D)).upload(sc.draw(t * n * D).reshape(t, n * D)))
+        k, v, q = tensors
+        outs = []
+        for fn in (hip.L.yx_attention_append_dev, hip.L.yx_attention_append_noalloc):
+            o = hip.tensor((t, hq * D))
+            tensors.append(o)
+            check_hip(fn(hip.ctx, sc.kv.h, 0, k.ptr, v.ptr, q.ptr, o.ptr, hq, hkv, 0,
+                         float(np.float32(1.0) / np.sqrt(np.float32(D)))))
+            hip.sync()
+            outs.append(o.numpy())
+        assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+    finally:
+        for x in tensors:
+            x.free()
         sc.kv.destroy()
