@@ -76,6 +76,9 @@ struct SubRef {
 
 static constexpr float kLog2e = 1.4426950408889634f;
 static constexpr int kD = 128;
+// Weights are taken relative to the running maximum, or to this where there is none yet: a
+// masked key (-inf) weighs 0 there too, and a NaN score stays NaN.
+static constexpr float kLowest = -3.40282347e+38f;
 static constexpr uint32_t kMaxChunks = 256;
 // Arrival counters (split-K hand-offs) sit one per 128-byte line, in uint32 units:
 // atomics to one line queue behind each other at its L2 channel.
@@ -251,7 +254,7 @@ __device__ __forceinline__ void merge_group(uint32_t g_r0, uint32_t g_nrows, uin
       }
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        if (c0 + j >= c_end || !(ml[j].y > 0.0f)) continue;  // past the range, or empty
+        if (c0 + j >= c_end || ml[j].y == 0.0f) continue;  // past the range, or empty (not a NaN sum)
         const float mn = fmaxf(mt, ml[j].x);
         const float r = __builtin_amdgcn_exp2f(mt - mn), wt = __builtin_amdgcn_exp2f(ml[j].x - mn);
         lt = lt * r + ml[j].y * wt;
@@ -284,7 +287,7 @@ __device__ __forceinline__ void merge_group(uint32_t g_r0, uint32_t g_nrows, uin
     if (part == 0) {
       for (uint32_t pp = 1; pp < parts; ++pp) {
         const float2 b = part_ml_lds[pp * span + pi];
-        if (!(b.y > 0.0f)) continue;
+        if (b.y == 0.0f) continue;
         const float4 ob = part_o_lds[pp * span + pi];
         const float mn = fmaxf(mt, b.x);
         const float r = __builtin_amdgcn_exp2f(mt - mn), wt = __builtin_amdgcn_exp2f(b.x - mn);
@@ -528,17 +531,17 @@ __global__ __launch_bounds__(64 * kWaves) void paged_attn_decode(
       }
       bmax = max_xor32(max_xor16(bmax));
       const float mn = fmaxf(m[t], bmax);
-      const bool live = mn != -INFINITY;
+      const float mf = fmaxf(mn, kLowest);
       float pr[8], rs = 0.0f;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        pr[i] = live ? __builtin_amdgcn_exp2f(x[i] - mn) : 0.0f;
+        pr[i] = __builtin_amdgcn_exp2f(x[i] - mf);
         rs += pr[i];
       }
       rs = sum_xor32(sum_xor16(rs));
       // Rescale only when some column's maximum moved (wave-uniform test).
       if (__builtin_amdgcn_ballot_w64(mn != m[t])) {
-        const float corr = live ? __builtin_amdgcn_exp2f(m[t] - mn) : 1.0f;
+        const float corr = __builtin_amdgcn_exp2f(m[t] - mf);
         l[t] *= corr;
 #pragma unroll
         for (int j = 0; j < 8; ++j) acc[t][j] *= corr;
@@ -615,17 +618,16 @@ __global__ __launch_bounds__(64 * kWaves) void paged_attn_decode(
     for (int w = 0; w < kWaves; ++w) mt = fmaxf(mt, sh.m[w][lr]);
     lt = 0.0f;
     o = float4{0, 0, 0, 0};
-    if (mt != -INFINITY) {
+    const float mf = fmaxf(mt, kLowest);
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w) {
-        const float wt = __builtin_amdgcn_exp2f(sh.m[w][lr] - mt);  // 0 for an empty wave
-        lt += sh.l[w][lr] * wt;
-        const float4 ow = sh.o[w][lr][qi];
-        o.x += ow.x * wt;
-        o.y += ow.y * wt;
-        o.z += ow.z * wt;
-        o.w += ow.w * wt;
-      }
+    for (int w = 0; w < kWaves; ++w) {
+      const float wt = __builtin_amdgcn_exp2f(sh.m[w][lr] - mf);  // 0 for an empty wave
+      lt += sh.l[w][lr] * wt;
+      const float4 ow = sh.o[w][lr][qi];
+      o.x += ow.x * wt;
+      o.y += ow.y * wt;
+      o.z += ow.z * wt;
+      o.w += ow.w * wt;
     }
   });
 }
@@ -837,16 +839,16 @@ __global__ __launch_bounds__(64 * kBalWaves) void paged_attn_decode_balanced(
     }
     bmax = max_xor32(max_xor16(bmax));
     const float mn = fmaxf(m, bmax);
-    const bool live = mn != -INFINITY;
+    const float mf = fmaxf(mn, kLowest);
     float pr[4], rs = 0.0f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      pr[i] = live ? __builtin_amdgcn_exp2f(x[i] - mn) : 0.0f;
+      pr[i] = __builtin_amdgcn_exp2f(x[i] - mf);
       rs += pr[i];
     }
     rs = sum_xor32(sum_xor16(rs));
     if (__builtin_amdgcn_ballot_w64(mn != m)) {
-      const float corr = live ? __builtin_amdgcn_exp2f(m - mn) : 1.0f;
+      const float corr = __builtin_amdgcn_exp2f(m - mf);
       l *= corr;
 #pragma unroll
       for (int j = 0; j < 8; ++j) acc[j] *= corr;
@@ -911,9 +913,9 @@ __global__ __launch_bounds__(64 * kBalWaves) void paged_attn_decode_balanced(
     for (uint32_t k = 0; k < nq; ++k) mt = fmaxf(mt, sh.m[k][lr]);
     lt = 0.0f;
     o = float4{0, 0, 0, 0};
-    if (mt == -INFINITY) return;
+    const float mf = fmaxf(mt, kLowest);
     for (uint32_t k = 0; k < nq; ++k) {
-      const float wt = __builtin_amdgcn_exp2f(sh.m[k][lr] - mt);  // 0 for an empty quad
+      const float wt = __builtin_amdgcn_exp2f(sh.m[k][lr] - mf);  // 0 for an empty quad
       lt += sh.l[k][lr] * wt;
       const float4 ow = sh.o[k][lr][qi];
       o.x += ow.x * wt;
@@ -1090,16 +1092,16 @@ __global__ __launch_bounds__(64 * kWideWaves) void paged_attn_decode_wide(
       }
       bmax = max_xor32(max_xor16(bmax));
       const float mn = fmaxf(m[t], bmax);
-      const bool live = mn != -INFINITY;
+      const float mf = fmaxf(mn, kLowest);
       float pr[4], rs = 0.0f;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        pr[i] = live ? __builtin_amdgcn_exp2f(x[i] - mn) : 0.0f;
+        pr[i] = __builtin_amdgcn_exp2f(x[i] - mf);
         rs += pr[i];
       }
       rs = sum_xor32(sum_xor16(rs));
       if (__builtin_amdgcn_ballot_w64(mn != m[t])) {
-        const float corr = live ? __builtin_amdgcn_exp2f(m[t] - mn) : 1.0f;
+        const float corr = __builtin_amdgcn_exp2f(m[t] - mf);
         l[t] *= corr;
 #pragma unroll
         for (int j = 0; j < 8; ++j) acc[t][j] *= corr;
@@ -1155,10 +1157,10 @@ __global__ __launch_bounds__(64 * kWideWaves) void paged_attn_decode_wide(
     for (int w = 0; w < kWideWaves; ++w) mt = fmaxf(mt, sh.m[w][lr]);
     lt = 0.0f;
     o = float4{0, 0, 0, 0};
-    if (mt == -INFINITY) return;
+    const float mf = fmaxf(mt, kLowest);
 #pragma unroll
     for (int w = 0; w < kWideWaves; ++w) {
-      const float wt = __builtin_amdgcn_exp2f(sh.m[w][lr] - mt);  // 0 for an empty wave
+      const float wt = __builtin_amdgcn_exp2f(sh.m[w][lr] - mf);  // 0 for an empty wave
       lt += sh.l[w][lr] * wt;
       const float4 ow = sh.o[w][lr][qi];
       o.x += ow.x * wt;
@@ -1319,16 +1321,16 @@ __global__ __launch_bounds__(64 * kWideWaves) void paged_attn_decode_f32(
     }
     bmax = max_xor32(max_xor16(bmax));
     const float mn = fmaxf(m, bmax);
-    const bool live = mn != -INFINITY;
+    const float mf = fmaxf(mn, kLowest);
     float pr[4], rs = 0.0f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      pr[i] = live ? __builtin_amdgcn_exp2f(x[i] - mn) : 0.0f;
+      pr[i] = __builtin_amdgcn_exp2f(x[i] - mf);
       rs += pr[i];
     }
     rs = sum_xor32(sum_xor16(rs));
     if (__builtin_amdgcn_ballot_w64(mn != m)) {
-      const float corr = live ? __builtin_amdgcn_exp2f(m - mn) : 1.0f;
+      const float corr = __builtin_amdgcn_exp2f(m - mf);
       l *= corr;
 #pragma unroll
       for (int j = 0; j < 8; ++j) acc[j] *= corr;
@@ -1372,10 +1374,10 @@ __global__ __launch_bounds__(64 * kWideWaves) void paged_attn_decode_f32(
     for (int w = 0; w < kWideWaves; ++w) mt = fmaxf(mt, sh.m[w][lr2]);
     lt = 0.0f;
     o = float4{0, 0, 0, 0};
-    if (mt == -INFINITY) return;
+    const float mf = fmaxf(mt, kLowest);
 #pragma unroll
     for (int w = 0; w < kWideWaves; ++w) {
-      const float wt = __builtin_amdgcn_exp2f(sh.m[w][lr2] - mt);
+      const float wt = __builtin_amdgcn_exp2f(sh.m[w][lr2] - mf);
       lt += sh.l[w][lr2] * wt;
       const float4 ow = sh.o[w][lr2][qi];
       o.x += ow.x * wt;

@@ -102,7 +102,7 @@ __device__ __forceinline__ void merge_tile(uint32_t r0, uint32_t nrows, uint32_t
       for (int j = 0; j < kGE; ++j)
 #pragma unroll
         for (int b = 0; b < kCB; ++b) {
-          if (c0 + b >= nch || !(ml[j][b].y > 0.0f)) continue;  // past the list, or empty
+          if (c0 + b >= nch || ml[j][b].y == 0.0f) continue;  // past the list, or empty (not a NaN sum)
           const float mn = fmaxf(mt[j], ml[j][b].x);
           const float r = __builtin_amdgcn_exp2f(mt[j] - mn), wt = __builtin_amdgcn_exp2f(ml[j][b].x - mn);
           lt[j] = lt[j] * r + ml[j][b].y * wt;
