@@ -62,6 +62,55 @@ def test_parts_match_f32_products(hip, ks, qs, vs, scale, bad, window):
         sc.kv.destroy()
 
 
+def _mantissas(rng, shape, low):
+    """Values in [1, 2) whose lower 16 bits are all but the largest (low), or zero."""
+    u = (0x3F80 + rng.integers(0, 128, shape)).astype(np.uint32) << 16
+    if low:
+        u |= (0xFF00 + rng.integers(0, 256, shape)).astype(np.uint32)
+    return u.view(np.float32)
+
+
+@pytest.mark.parametrize("ctx", [64, 1000])
+def test_parts_leave_nothing_out_on_one_side(hip, ctx):
+    """Values just below a bf16 step, where the products of small parts that are left out
+    are largest. In scores: keys with such values against keys that are bf16 exactly, told
+    apart by V = +-1, so that a loss of one kind shows in every output; not further off 64
+    bits than f32 products. In V: the mean error below 2^-26 of the values, the largest that
+    one output's left-out products may reach."""
+    hq, hkv, rows = 8, 2, 64
+    rng = np.random.default_rng(1)
+    even = (np.arange(ctx) % 2 == 0)[:, None, None]
+    kv = (ctx, hkv, D)
+    worst = _mantissas(rng, kv, True)
+    passes = [(np.where(even, worst, _mantissas(rng, kv, False)), np.broadcast_to(np.where(even, 1.0, -1.0), kv),
+               _mantissas(rng, (rows, hq * D), True)),
+              (rng.standard_normal(kv), worst, rng.standard_normal((rows, hq * D)))]
+    err = {}
+    for i, (k, v, q) in enumerate(passes):
+        for waves in (8, 4):
+            sc = Scenario(hip, pages=ctx // 32 + 8, page=32, hkv=hkv, pool_seed=5, f32=True)
+            try:
+                seq = sc.cache.new_seq()
+                pr = sc.run_pass([(seq, ctx)])
+                k, v, q = (np.ascontiguousarray(x, np.float32) for x in (k, v, q))
+                hip.append(sc.kv, 0, k, v)
+                sc.orc[0].store(pr.meta.kv_slot, k.reshape(ctx, -1), v.reshape(ctx, -1))
+                pr.meta.pos, pr.meta.pt_off, pr.meta.kv_slot, pr.meta.ids = (
+                    x[-rows:] for x in (pr.meta.pos, pr.meta.pt_off, pr.meta.kv_slot, pr.meta.ids))
+                hip.begin_pass(pr.meta)
+                hip.set_option("prefill_min_rows", 1)
+                hip.set_option("prefill_f32_waves", waves)
+                got = hip.attend(sc.kv, 0, q, hq)
+                want = sc.orc[0].attend_f64(q, hq, pr.meta.pos, pr.meta.pt_off, pr.meta.pages)
+                err[i, waves] = got - want
+            finally:
+                hip.set_option("prefill_min_rows", 0)
+                hip.set_option("prefill_f32_waves", 0)
+                sc.kv.destroy()
+    assert np.linalg.norm(err[0, 8]) <= np.linalg.norm(err[0, 4])
+    assert abs(err[1, 8].mean()) < 2.0 ** -26  # V is in [1, 2)
+
+
 @pytest.mark.parametrize("rows,prior,hq,hkv", [
     (8, 4096, 16, 4),    # tiles with a quarter of their rows, partial slots of 32
     (5, 1500, 12, 4),    # 15 logical rows: stays decode items

@@ -280,12 +280,29 @@ __device__ __forceinline__ void prefill_f32_exact(
   finish_tile<W>(it, kh, G, hq, hkv, out, ro, rml, counters, part_rows);
 }
 
+// Two f32 values as three bf16 parts each, packed as split_bf16x3 does, but cut to nearest:
+// |mid| is at most 2^-8 and |lo| 2^-16 of the value (2^-9 and 2^-18 of its power of two),
+// either sign, where truncation gives up to 2^-7 and 2^-15, all of the value's sign. The same
+// number of instructions. |f| below 0x1.ffp127 (above, hi is infinite).
+__device__ __forceinline__ void split_bf16x3_nearest(float f0, float f1, uint32_t& h, uint32_t& m, uint32_t& l) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  h = __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{f0, f1}, bf16x2));
+  const float r0 = f0 - __uint_as_float(h << 16), r1 = f1 - __uint_as_float(h & 0xffff0000u);
+  m = __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{r0, r1}, bf16x2));
+  const uint32_t s0 = __float_as_uint(r0 - __uint_as_float(m << 16));
+  const uint32_t s1 = __float_as_uint(r1 - __uint_as_float(m & 0xffff0000u));
+  l = __builtin_amdgcn_perm(s1, s0, 0x07060302);  // at most 8 bits are left: exact
+}
+
 // The tile of 128 logical rows on bf16 products: K, V, q and P each as three bf16 parts
-// (hi, mid, lo: the 24 significand bits cut by truncation, exactly), and of the nine
-// products of two such numbers the six down to 2^-16 of the largest; what is left out is
-// below 2^-23 of |k q| (2^-25 on average), less than the rounding of the f32 sums. bf16 has
-// f32's range, so every finite value is served, and f32 accumulation as before. Six
-// v_mfma_f32_16x16x32_bf16 take 96 cycles where eight v_mfma_f32_16x16x4_f32 take 256.
+// (hi, mid, lo: the 24 significand bits cut to nearest, exactly), and of the nine products
+// of two such numbers the six down to 2^-18 of the largest; what is left out (mid lo, lo mid,
+// lo lo) is below 2^-26 of 2^(the exponents of k and q), either sign, half a rounding of the
+// product to f32. (Parts cut by truncation lose up to 2^-21 of |k q|, always towards zero:
+// on values just below a bf16 step, out of 1000 keys, 2.4e-5 off 64 bits where f32 products
+// are 2.7e-6 and these 7e-7 off.) bf16 has f32's range, so every finite value is served, and
+// f32 accumulation as before. Six v_mfma_f32_16x16x32_bf16 take 96 cycles where eight
+// v_mfma_f32_16x16x4_f32 take 256.
 // Returns false, with nothing written, where parts would not do: an infinity (0 * inf in a
 // product of parts) or a NaN (a masked key's reaches the rows of its 32 keys here, of 16 in
 // f32 products); K, q or the scale so large that parts below bf16's range matter to a
@@ -357,7 +374,7 @@ __device__ __forceinline__ bool prefill_f32_parts(
     for (int e = 0; e < 4; ++e) {
       __asm__("v_maximum3_f32 %0, %0, |%1|, |%2|" : "+v"(top) : "v"(v[2 * e]), "v"(v[2 * e + 1]));
       uint32_t h, m, l;
-      split_bf16x3<false>(v[2 * e], v[2 * e + 1], h, m, l);
+      split_bf16x3_nearest(v[2 * e], v[2 * e + 1], h, m, l);
       p[0][e] = h;
       p[1][e] = m;
       p[2][e] = l;
@@ -476,7 +493,7 @@ __device__ __forceinline__ bool prefill_f32_parts(
       const float a = __builtin_amdgcn_exp2f(x[2 * e] - m), b = __builtin_amdgcn_exp2f(x[2 * e + 1] - m);
       lsum += a + b;
       uint32_t hh, mm, ll;
-      split_bf16x3<false>(a, b, hh, mm, ll);
+      split_bf16x3_nearest(a, b, hh, mm, ll);
       pw[0][e] = hh;
       pw[1][e] = mm;
       pw[2][e] = ll;
@@ -535,7 +552,7 @@ __device__ __forceinline__ bool prefill_f32_parts(
   for (int s = 1; s < 16; s <<= 1) vall = fmaxf(vall, __shfl_xor(vall, s));
   float* const tops = reinterpret_cast<float*>(lds);
   if (lane == 0) tops[wave] = vall;
-  const bool huge = __syncthreads_or(!(big < 0x1p70f) || !(vbig < INFINITY));
+  const bool huge = __syncthreads_or(!(big < 0x1p70f) || !(vbig < 0x1.ffp127f));
   float vmax = 0.0f;
 #pragma unroll
   for (int w = 0; w < kPf32Waves; ++w) vmax = fmaxf(vmax, tops[w]);
