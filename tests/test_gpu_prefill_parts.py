@@ -111,6 +111,32 @@ def test_parts_leave_nothing_out_on_one_side(hip, ctx):
     assert abs(err[1, 8].mean()) < 2.0 ** -26  # V is in [1, 2)
 
 
+@pytest.mark.parametrize("low", [-90, -108, -112, -118])
+def test_small_values_beside_large_ones(hip, low):
+    """V whose upper dims are 2^low of the lower ones, in a tile with both: each output as
+    exact as f32 products give it."""
+    hq, hkv, rows = 8, 2, 300
+    sc = Scenario(hip, pages=rows // 32 + 8, page=32, hkv=hkv, pool_seed=5, f32=True)
+    try:
+        seq = sc.cache.new_seq()
+        pr = sc.run_pass([(seq, rows)])
+        k, v = (sc.draw(rows * hkv * D).reshape(rows, hkv, D) for _ in range(2))
+        v[:, :, 64:] *= np.float32(2.0) ** low
+        q = sc.draw(rows * hq * D).reshape(rows, hq * D)
+        hip.append(sc.kv, 0, k, v)
+        sc.orc[0].store(pr.meta.kv_slot, k.reshape(rows, -1), v.reshape(rows, -1))
+        want = sc.orc[0].attend_f64(q, hq, pr.meta.pos, pr.meta.pt_off, pr.meta.pages)
+        hip.set_option("prefill_min_rows", 1)
+        got = hip.attend(sc.kv, 0, q, hq)
+        for half in (slice(0, 64), slice(64, 128)):
+            a, b = (x.reshape(rows, hq, D)[..., half].astype(np.float64) * 2.0 ** -low for x in (got, want))
+            # f32 products are 1.4e-7 off; parts that lose V's low bits 2.5e-7 (2^-112), 9e-6 (2^-118).
+            assert np.linalg.norm(a - b) < 2e-7 * np.linalg.norm(b)
+    finally:
+        hip.set_option("prefill_min_rows", 0)
+        sc.kv.destroy()
+
+
 @pytest.mark.parametrize("rows,prior,hq,hkv", [
     (8, 4096, 16, 4),    # tiles with a quarter of their rows, partial slots of 32
     (5, 1500, 12, 4),    # 15 logical rows: stays decode items

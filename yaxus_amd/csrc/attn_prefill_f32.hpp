@@ -283,8 +283,10 @@ __device__ __forceinline__ void prefill_f32_exact(
 // Two f32 values as three bf16 parts each, packed as split_bf16x3 does, but cut to nearest:
 // |mid| is at most 2^-8 and |lo| 2^-16 of the value (2^-9 and 2^-18 of its power of two),
 // either sign, where truncation gives up to 2^-7 and 2^-15, all of the value's sign. The same
-// number of instructions. |f| below 0x1.ffp127 (above, hi is infinite).
-__device__ __forceinline__ void split_bf16x3_nearest(float f0, float f1, uint32_t& h, uint32_t& m, uint32_t& l) {
+// number of instructions. |f| below 0x1.ffp127 (above, hi is infinite). `lost` gathers in its
+// lower half the bits below bf16's range, 2^-133 (of values below 2^-110 only).
+__device__ __forceinline__ void split_bf16x3_nearest(float f0, float f1, uint32_t& h, uint32_t& m, uint32_t& l,
+                                                     uint32_t& lost) {
   typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
   h = __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{f0, f1}, bf16x2));
   const float r0 = f0 - __uint_as_float(h << 16), r1 = f1 - __uint_as_float(h & 0xffff0000u);
@@ -292,6 +294,7 @@ __device__ __forceinline__ void split_bf16x3_nearest(float f0, float f1, uint32_
   const uint32_t s0 = __float_as_uint(r0 - __uint_as_float(m << 16));
   const uint32_t s1 = __float_as_uint(r1 - __uint_as_float(m & 0xffff0000u));
   l = __builtin_amdgcn_perm(s1, s0, 0x07060302);  // at most 8 bits are left: exact
+  lost |= s0 | s1;
 }
 
 // The tile of 128 logical rows on bf16 products: K, V, q and P each as three bf16 parts
@@ -306,9 +309,10 @@ __device__ __forceinline__ void split_bf16x3_nearest(float f0, float f1, uint32_
 // Returns false, with nothing written, where parts would not do: an infinity (0 * inf in a
 // product of parts) or a NaN (a masked key's reaches the rows of its 32 keys here, of 16 in
 // f32 products); K, q or the scale so large that parts below bf16's range matter to a
-// score (at most 2^-126 * 2^70 * 2^7 dims * 2^20, 2^-29); a tile whose V is all below 2^-90
-// (with one value above it, what its parts lose is below 2^-36 of that). The caller then
-// runs the f32 products.
+// score (at most 2^-133 * 2^70 * 2^7 dims * 2^20, 2^-36); a value of V with bits below that
+// range, 2^-133 (one of 2^-110 keeps all 24; lost, an output made of such values alone would
+// be as far off: 5.7e-4 at 2^-124). The caller then runs the f32 products. (A weight's bits
+// below 2^-133 are dropped: the exponential itself gives 0 below 2^-126.)
 //
 // Stages of 32 keys: each thread reads 8 dims of one key of K and of V (f32) into
 // registers, one stage ahead, cuts them into parts and stores those to one of two LDS
@@ -368,13 +372,14 @@ __device__ __forceinline__ bool prefill_f32_parts(
     vr[1] = *reinterpret_cast<const float4*>(vs + 4);
   };
   float big = 0.0f, vbig = 0.0f;  // largest |K|, |q| and |V| met by this thread, or NaN
-  auto split8 = [&](const float4& a, const float4& b, u32x4 (&p)[3], float& top) __attribute__((always_inline)) {
+  uint32_t vlost = 0, unused = 0;
+  auto split8 = [&](const float4& a, const float4& b, u32x4 (&p)[3], float& top, uint32_t& lost) __attribute__((always_inline)) {
     const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       __asm__("v_maximum3_f32 %0, %0, |%1|, |%2|" : "+v"(top) : "v"(v[2 * e]), "v"(v[2 * e + 1]));
       uint32_t h, m, l;
-      split_bf16x3_nearest(v[2 * e], v[2 * e + 1], h, m, l);
+      split_bf16x3_nearest(v[2 * e], v[2 * e + 1], h, m, l, lost);
       p[0][e] = h;
       p[1][e] = m;
       p[2][e] = l;
@@ -382,10 +387,10 @@ __device__ __forceinline__ bool prefill_f32_parts(
   };
   auto store = [&](uint32_t slot) __attribute__((always_inline)) {
     u32x4 p[3];
-    split8(kr[0], kr[1], p, big);
+    split8(kr[0], kr[1], p, big, unused);
 #pragma unroll
     for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x4*>(k_dst + slot * kSlot + i * 8192) = p[i];
-    split8(vr[0], vr[1], p, vbig);
+    split8(vr[0], vr[1], p, vbig, vlost);
 #pragma unroll
     for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x4*>(v_dst + slot * kSlot + i * 8192) = p[i];
   };
@@ -408,7 +413,7 @@ __device__ __forceinline__ bool prefill_f32_parts(
       float4 a = *reinterpret_cast<const float4*>(qp + 32 * pp), b = *reinterpret_cast<const float4*>(qp + 32 * pp + 4);
       if (!has) a = b = float4{0, 0, 0, 0};
       u32x4 p[3];
-      split8(a, b, p, big);
+      split8(a, b, p, big, unused);
 #pragma unroll
       for (int i = 0; i < 3; ++i) qf[i][pp] = __builtin_bit_cast(bf16x8, p[i]);
     }
@@ -493,7 +498,7 @@ __device__ __forceinline__ bool prefill_f32_parts(
       const float a = __builtin_amdgcn_exp2f(x[2 * e] - m), b = __builtin_amdgcn_exp2f(x[2 * e + 1] - m);
       lsum += a + b;
       uint32_t hh, mm, ll;
-      split_bf16x3_nearest(a, b, hh, mm, ll);
+      split_bf16x3_nearest(a, b, hh, mm, ll, unused);
       pw[0][e] = hh;
       pw[1][e] = mm;
       pw[2][e] = ll;
@@ -546,17 +551,7 @@ __device__ __forceinline__ bool prefill_f32_parts(
     lds_barrier();
   }
   // Values that parts don't serve: over to f32 products.
-  const float vtop = max_xor32(max_xor16(vbig));
-  float vall = vtop;
-#pragma unroll
-  for (int s = 1; s < 16; s <<= 1) vall = fmaxf(vall, __shfl_xor(vall, s));
-  float* const tops = reinterpret_cast<float*>(lds);
-  if (lane == 0) tops[wave] = vall;
-  const bool huge = __syncthreads_or(!(big < 0x1p70f) || !(vbig < 0x1.ffp127f));
-  float vmax = 0.0f;
-#pragma unroll
-  for (int w = 0; w < kPf32Waves; ++w) vmax = fmaxf(vmax, tops[w]);
-  if (huge || (vmax > 0.0f && vmax < 0x1p-90f)) {
+  if (__syncthreads_or(!(big < 0x1p70f) || !(vbig < 0x1.ffp127f) || (vlost & 0xffffu) != 0)) {
     __syncthreads();
     return false;
   }
