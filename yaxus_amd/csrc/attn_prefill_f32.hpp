@@ -164,10 +164,9 @@ __device__ __forceinline__ void prefill_f32_exact(
   const int first_key = static_cast<int>(it.blk0 * 16);
   const int key_end = static_cast<int>(it.blk1 * 16);
 
-  // As in the f16 kernel, the running maximum starts at a finite floor: masked scores
-  // (-inf) give P = 0 and a column's first key rescales its zero state away.
-  constexpr float kFloor = -1.0e30f;
-  float m = kFloor, lsum = 0.0f;
+  // The running maximum starts at the lowest finite value (f32 K and q may score down to it):
+  // masked scores (-inf) give P = 0 and a column's first key rescales its zero state away.
+  float m = kLowest, lsum = 0.0f;
   floatx4 acc[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) acc[j] = floatx4{0, 0, 0, 0};
@@ -187,7 +186,7 @@ __device__ __forceinline__ void prefill_f32_exact(
     float4 vf[8];
 #pragma unroll
     for (int r = 0; r < 8; ++r) vf[r] = vb[r * 64 + lane];
-    float x[4], bmax = kFloor;
+    float x[4], bmax = kLowest;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float s = ((sp[0][i] + sp[1][i]) + (sp[2][i] + sp[3][i])) * scale_log2;
@@ -433,8 +432,7 @@ __device__ __forceinline__ bool prefill_f32_parts(
   const int first_key = static_cast<int>(it.blk0 * 16);
   const int key_end = static_cast<int>(it.blk1 * 16);
 
-  constexpr float kFloor = -1.0e30f;
-  float m = kFloor, lsum = 0.0f;
+  float m = kLowest, lsum = 0.0f;
   floatx4 acc[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) acc[j] = floatx4{0, 0, 0, 0};
@@ -471,7 +469,7 @@ __device__ __forceinline__ bool prefill_f32_parts(
           to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[b][kPa[t]], qf[kPb[t]][pp], to, 0, 0, 0);
         }
     }
-    float x[8], bmax = kFloor;
+    float x[8], bmax = kLowest;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const float s = (sc[e >> 2][e & 3] + sm[e >> 2][e & 3]) * scale_log2;
