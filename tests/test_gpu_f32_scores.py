@@ -48,3 +48,29 @@ def test_scores_near_the_ends_of_the_range(hip, waves, size):
         hip.set_option("prefill_min_rows", 0)
         hip.set_option("prefill_f32_waves", 0)
         sc.kv.destroy()
+
+
+@pytest.mark.parametrize("tiles", [0, 1])
+def test_values_near_the_end_of_the_range(hip, tiles):
+    """V of 2^119, and keys whose scores grow by less than a tile's maximum lags behind
+    (2^8): the weights stay below 1 as on the CPU backend, so 240 keys' sum is finite."""
+    hq, hkv, n = 8, 2, 240
+    sc = Scenario(hip, pages=n // 16 + 4, page=16, hkv=hkv, pool_seed=3, f32=True)
+    try:
+        seq = sc.cache.new_seq()
+        pr = sc.run_pass([(seq, n)])
+        k = np.zeros((n, hkv, D), np.float32)
+        k[64:, :, 9] = 5 * np.sqrt(np.float32(D))
+        v = (1 + np.abs(sc.draw(n * hkv * D).reshape(n, hkv, D)) / 8) * np.float32(2.0 ** 119)
+        q = np.zeros((n, hq, D), np.float32)
+        q[:, :, 9] = 1
+        q = q.reshape(n, -1)
+        hip.append(sc.kv, 0, k, v)
+        sc.orc[0].store(pr.meta.kv_slot, k.reshape(n, -1), v.reshape(n, -1))
+        hip.set_option("prefill_min_rows", 1 if tiles else 1 << 20)
+        got = hip.attend(sc.kv, 0, q, hq)
+        want = sc.orc[0].attend_f64(q, hq, pr.meta.pos, pr.meta.pt_off, pr.meta.pages)
+        assert np.abs(got - want).max() < 2e-6 * 2.0 ** 119
+    finally:
+        hip.set_option("prefill_min_rows", 0)
+        sc.kv.destroy()

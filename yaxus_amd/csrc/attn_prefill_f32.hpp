@@ -167,6 +167,9 @@ __device__ __forceinline__ void prefill_f32_exact(
   // The running maximum starts at the lowest finite value (f32 K and q may score down to it):
   // masked scores (-inf) give P = 0 and a column's first key rescales its zero state away.
   float m = kLowest, lsum = 0.0f;
+  // How far the maximum may lag. Tiles that parts handed over may have V so large that only
+  // weights of at most 1 keep its sums finite.
+  constexpr float kLag = W == kPf32Waves ? 0.0f : kLazyRescale;
   floatx4 acc[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) acc[j] = floatx4{0, 0, 0, 0};
@@ -200,7 +203,7 @@ __device__ __forceinline__ void prefill_f32_exact(
       bmax = fmaxf(bmax, x[i]);
     }
     const float mnew = fmaxf(m, max_xor32(max_xor16(bmax)));
-    if (__builtin_amdgcn_ballot_w64(mnew > m + kLazyRescale)) {  // wave-uniform
+    if (__builtin_amdgcn_ballot_w64(mnew > m + kLag)) {  // wave-uniform
       const float corr = __builtin_amdgcn_exp2f(m - mnew);
       lsum *= corr;
 #pragma unroll
@@ -282,7 +285,7 @@ __device__ __forceinline__ void prefill_f32_exact(
 // Two f32 values as three bf16 parts each, packed as split_bf16x3 does, but cut to nearest:
 // |mid| is at most 2^-8 and |lo| 2^-16 of the value (2^-9 and 2^-18 of its power of two),
 // either sign, where truncation gives up to 2^-7 and 2^-15, all of the value's sign. The same
-// number of instructions. |f| below 0x1.ffp127 (above, hi is infinite). `lost` gathers in its
+// number of instructions. |f| below 0x1.ffp127 (from there on hi is infinite). `lost` gathers in its
 // lower half the bits below bf16's range, 2^-133 (of values below 2^-110 only).
 __device__ __forceinline__ void split_bf16x3_nearest(float f0, float f1, uint32_t& h, uint32_t& m, uint32_t& l,
                                                      uint32_t& lost) {
@@ -310,7 +313,8 @@ __device__ __forceinline__ void split_bf16x3_nearest(float f0, float f1, uint32_
 // f32 products); K, q or the scale so large that parts below bf16's range matter to a
 // score (at most 2^-133 * 2^70 * 2^7 dims * 2^20, 2^-36); a value of V with bits below that
 // range, 2^-133 (one of 2^-110 keeps all 24; lost, an output made of such values alone would
-// be as far off: 5.7e-4 at 2^-124). The caller then runs the f32 products. (A weight's bits
+// be as far off: 5.7e-4 at 2^-124); V of 2^100 and more (weights of up to 2^kLazyRescale times
+// many such values might overflow where weights of at most 1 do not). The caller then runs the f32 products. (A weight's bits
 // below 2^-133 are dropped: the exponential itself gives 0 below 2^-126.)
 //
 // Stages of 32 keys: each thread reads 8 dims of one key of K and of V (f32) into
@@ -549,7 +553,7 @@ __device__ __forceinline__ bool prefill_f32_parts(
     lds_barrier();
   }
   // Values that parts don't serve: over to f32 products.
-  if (__syncthreads_or(!(big < 0x1p70f) || !(vbig < 0x1.ffp127f) || (vlost & 0xffffu) != 0)) {
+  if (__syncthreads_or(!(big < 0x1p70f) || !(vbig < 0x1p100f) || (vlost & 0xffffu) != 0)) {
     __syncthreads();
     return false;
   }
