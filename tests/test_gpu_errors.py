@@ -7,6 +7,7 @@ from types import SimpleNamespace
 import numpy as np
 import pytest
 
+from tests.scenario import Scenario
 from yaxus_amd._lib import YxError
 
 pytestmark = pytest.mark.gpu
@@ -132,3 +133,17 @@ def test_python_mirror_rejects_short_device_tensors(hip, kv):
     finally:
         for t in (q, out, k, v):
             t.free()
+
+
+@pytest.mark.parametrize("hq,batch,rows,prior", [(17, 1, 64, 9000), (17, 8, 64, 529), (17, 40, 4, 2000)])
+def test_f32_more_q_heads_than_an_item_holds(hip, hq, batch, rows, prior):
+    """More than 16 q heads per KV head: refused, also where tiles would be the faster kernel."""
+    sc = Scenario(hip, pages=batch * (-(-(rows + prior) // 64)) + 4, page=64, hkv=1, pool_seed=13, f32=True)
+    try:
+        seqs = [sc.cache.new_seq() for _ in range(batch)]
+        sc.run_pass([(s, prior) for s in seqs])
+        sc.run_pass([(s, rows) for s in seqs])
+        with pytest.raises(YxError, match="more than 16 query heads"):
+            hip.attend(sc.kv, 0, np.zeros((batch * rows, hq * D), np.float32), hq)
+    finally:
+        sc.kv.destroy()

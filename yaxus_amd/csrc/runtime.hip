@@ -569,8 +569,10 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
     use_prefill = max_rows * G > 16 && decode_us > prefill_us;
     // Decode items serve a pass this short through the entry point that allocates nothing:
     // tiles take it only if their partials fit that scratch too (not, for one, those of
-    // 4 x 64 chunks of 128 rows after 28000 keys).
+    // 4 x 64 chunks of 128 rows after 28000 keys). More q heads per KV head than a decode
+    // item holds: such a pass is refused, whichever kernel would be faster.
     must_fit = decode_us <= 95.0 + 2.4 * max_keys / 1024.0;
+    if (G > 16) use_prefill = max_rows * G > 16 && !must_fit;
   } else {
     size_t tiles = 0;
     for (const Group& g : c->groups) tiles += (g.n * G + yx::kPrefillRows - 1) / yx::kPrefillRows;
