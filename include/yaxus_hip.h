@@ -45,7 +45,8 @@ const char* yx_last_error(void);
 int yx_device_count(int* n);
 
 /* A context: one device, one stream, the current pass's metadata and the scratch
- * space of the attention (split-K partials and arrival counters). */
+ * space of the attention (split-K partials and arrival counters) and of matmuls (32 MiB
+ * from the start for passes of many rows). */
 int yx_ctx_create(int device, yx_ctx** out);
 int yx_ctx_destroy(yx_ctx* ctx);
 int yx_sync(yx_ctx* ctx);

@@ -75,3 +75,52 @@ def test_graph_replays_match_eager(hip, kind):
     for t in (q, k, v, *outs):
         t.free()
     sc.kv.destroy()
+
+
+def _matmul_operands(hip, t, k, n):
+    x, w, out = hip.tensor((t, k)), hip.tensor((n, k), np.uint16), hip.tensor((t, n))
+    hip.fill_normal(x.ptr, t * k, False, 5, t)
+    w.upload(np.random.default_rng(n).integers(0x3C00, 0x3E00, (n, k)).astype(np.uint16))
+    return x, w, out
+
+
+@pytest.mark.parametrize("t", [80, 600, 1030])  # tiles of three shapes, k split in four and in two
+def test_matmul_of_many_rows_is_captured_without_an_earlier_call(t):
+    from yaxus_amd.backend import HipBackend
+
+    hip = HipBackend(0)
+    try:
+        x, w, out = _matmul_operands(hip, t, 2048, 2048)
+        hip.graph_begin()
+        hip.matmul_bf16(x, w, out=out)
+        hip.graph_end()
+        got = []
+        for rep in range(3):
+            hip.fill_normal(out.ptr, out.nbytes // 4, False, 99, rep << 32)
+            hip.sync()
+            hip.graph_launch()
+            got.append(out.numpy())
+            hip.fill_normal(out.ptr, out.nbytes // 4, False, 98, rep << 32)
+            hip.matmul_bf16(x, w, out=out)
+            assert np.array_equal(got[-1].view(np.uint32), out.numpy().view(np.uint32)), f"replay {rep}"
+    finally:
+        hip.close()
+
+
+def test_matmul_of_many_rows_leaves_graphs_valid():
+    from yaxus_amd.backend import HipBackend
+
+    hip = HipBackend(0)
+    try:
+        few, many = _matmul_operands(hip, 8, 2048, 2048), _matmul_operands(hip, 1030, 2048, 2048)
+        hip.matmul_bf16(few[0], few[1], out=few[2])
+        want = few[2].numpy()
+        hip.graph_begin()
+        hip.matmul_bf16(few[0], few[1], out=few[2])
+        hip.graph_end()
+        hip.matmul_bf16(many[0], many[1], out=many[2])
+        hip.fill_normal(few[2].ptr, few[2].nbytes // 4, False, 99, 0)
+        hip.graph_launch()
+        assert np.array_equal(few[2].numpy().view(np.uint32), want.view(np.uint32))
+    finally:
+        hip.close()

@@ -346,6 +346,10 @@ struct yx_ctx {
   DevBuf part_o, part_ml, counters, io_a, io_b, io_c, io_q;
   DevBuf am_keys, am_counters;  // argmax: per-slice keys, per-row arrival counters
   DevBuf mm_part, mm_counters;  // matmul: per-k-part output tiles, per-tile arrival counters
+  // The same for matmul_bf16_tiles: the most it splits into, allocated with the context. So
+  // its calls need no earlier one to be captured, and (unlike the buffers counted in
+  // buffer_gens) leave captured graphs valid.
+  DevBuf mt_part, mt_counters;
   // options
   long target_waves = 0;  // 0: one work item per CU
   int cus = 256;
@@ -1451,10 +1455,10 @@ int qk_rope_impl(yx_ctx* c, yx_kv* kv, size_t layer, const yx::QkvIn& in, size_t
   return prof_end(c, YX_KERNEL_QK_ROPE, e0);
 }
 
-// Scratch of a matmul split along k: ks partial tiles of `elems` f32 per output tile and
-// one arrival counter per tile.
-int matmul_scratch(yx_ctx* c, size_t tiles, size_t ks, size_t elems) {
-  const size_t part = tiles * ks * elems * 4, cnt = tiles * 4 * yx::kCounterStride;
+// Scratch of matmul_bf16_rows split along k: ks partial tiles of 16 x 16 f32 per output tile
+// and one arrival counter per tile.
+int matmul_scratch(yx_ctx* c, size_t tiles, size_t ks) {
+  const size_t part = tiles * ks * 1024, cnt = tiles * 4 * yx::kCounterStride;
   if (c->capturing && (c->mm_part.cap < part || c->mm_counters.cap < cnt))
     return fail(YX_ERR_INVALID, "run the call once before capturing it (its scratch is allocated then)");
   if (part > 0xffffffffu) return fail(YX_ERR_UNSUPPORTED, "matmul dimensions too large");
@@ -1496,6 +1500,24 @@ bool matmul_stream(yx_ctx* c, const float* x, const uint16_t* w, float* out, uin
   }
 }
 
+// The shapes of matmul_bf16_tiles.
+struct MatmulShape {
+  uint32_t tm, tn, per_cu;  // workgroups per CU
+  double stage_us;          // per 32 k, with per_cu workgroups on a CU
+};
+constexpr MatmulShape kMatmulShapes[] = {{128, 256, 1, 1.22}, {128, 128, 1, 0.75}, {64, 128, 1, 0.46}, {64, 64, 2, 0.56}};
+
+// Its scratch, for splits of at most one round of workgroups (32 MiB on 256 CUs).
+int matmul_tiles_scratch(yx_ctx* c) {
+  size_t part = 0, slots = 0;
+  for (const MatmulShape& sh : kMatmulShapes) {
+    slots = std::max(slots, static_cast<size_t>(sh.per_cu) * c->cus);
+    part = std::max(part, static_cast<size_t>(sh.per_cu) * c->cus * sh.tm * sh.tn * 4);
+  }
+  if (int rc = c->mt_part.ensure(part, c->stream)) return rc;
+  return c->mt_counters.ensure(slots * 4 * yx::kCounterStride, c->stream, true);
+}
+
 // Many rows: LDS tiles. The tile shape and the split of k with the smallest estimated
 // time: rounds of workgroups times a workgroup's time, its stages of 32 k times the
 // shape's cost per stage (all CUs busy, measured over t 20-4096, k 1536-3072, n
@@ -1505,17 +1527,12 @@ bool matmul_stream(yx_ctx* c, const float* x, const uint16_t* w, float* out, uin
 // us, 128 x 128 114, 64 x 128 123; t 512: 64 x 128 split in two 22.3, 128 x 128 in four
 // 22.9, 128 x 256 in two 45; t 80: 64 x 64 in four 12.0, 64 x 128 in eight 12.7).
 int matmul_tiled(yx_ctx* c, const float* x, const uint16_t* w, float* out, uint32_t t, uint32_t k, uint32_t n) {
-  struct Shape {
-    uint32_t tm, tn, per_cu;  // workgroups per CU
-    double stage_us;          // per 32 k, with per_cu workgroups on a CU
-  };
-  static constexpr Shape kShapes[] = {{128, 256, 1, 1.22}, {128, 128, 1, 0.75}, {64, 128, 1, 0.46}, {64, 64, 2, 0.56}};
   const uint32_t steps = (k + 31) / 32;
   int best = 0;
   uint32_t best_ks = 1;
   double best_us = 1e30;
   for (int s = 0; s < 4; ++s) {
-    const Shape& sh = kShapes[s];
+    const MatmulShape& sh = kMatmulShapes[s];
     const uint64_t tiles = static_cast<uint64_t>((t + sh.tm - 1) / sh.tm) * ((n + sh.tn - 1) / sh.tn);
     const uint64_t slots = static_cast<uint64_t>(sh.per_cu) * c->cus;
     for (uint32_t ks = 1; ks <= 8 && (ks == 1 || (steps / ks >= 8 && tiles * ks <= slots)); ks *= 2) {
@@ -1532,15 +1549,13 @@ int matmul_tiled(yx_ctx* c, const float* x, const uint16_t* w, float* out, uint3
       }
     }
   }
-  const Shape& sh = kShapes[best];
+  const MatmulShape& sh = kMatmulShapes[best];
   const size_t tiles = static_cast<size_t>((t + sh.tm - 1) / sh.tm) * ((n + sh.tn - 1) / sh.tn);
   if (tiles > 0x7fffffff) return fail(YX_ERR_UNSUPPORTED, "matmul dimensions too large");
-  int rc;
-  if (best_ks > 1 && (rc = matmul_scratch(c, tiles, best_ks, sh.tm * sh.tn))) return rc;
   const auto go = [&](auto* kern) {
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(tiles), best_ks), dim3(yx::kMatmulThreads), 0, c->stream, x,
-                       w, out, t, k, n, static_cast<yx::f32x4*>(c->mm_part.p),
-                       static_cast<uint32_t>(c->mm_part.cap), static_cast<uint32_t*>(c->mm_counters.p));
+                       w, out, t, k, n, static_cast<yx::f32x4*>(c->mt_part.p),
+                       static_cast<uint32_t>(c->mt_part.cap), static_cast<uint32_t*>(c->mt_counters.p));
   };
   switch (best) {
     case 0: go(yx::matmul_bf16_tiles<yx::MatmulTileA>); break;
@@ -1590,7 +1605,9 @@ int yx_ctx_create(int device, yx_ctx** out) {
     delete c;
     return fail(YX_ERR_HIP, std::string("context set-up: ") + hipGetErrorString(e));
   }
-  if (int rc = scratch_init(device, c->stream)) {
+  int rc = scratch_init(device, c->stream);
+  if (!rc) rc = matmul_tiles_scratch(c);
+  if (rc) {
     yx_ctx_destroy(c);
     return rc;
   }
@@ -1615,6 +1632,7 @@ int yx_ctx_destroy(yx_ctx* c) {
   for (DevBuf& b : c->spare) b.release();
   c->spare.clear();
   for (DevBuf* b : {&c->d_meta, &c->d_pages, &c->am_keys, &c->am_counters, &c->mm_part, &c->mm_counters,
+                    &c->mt_part, &c->mt_counters,
                     &c->part_o, &c->part_ml, &c->counters,
                     &c->io_a, &c->io_b, &c->io_c, &c->io_q})
     b->release();
@@ -2270,7 +2288,7 @@ int yx_matmul_bf16_dev(yx_ctx* c, const float* x, const uint16_t* w, float* out,
   size_t ks = std::max<size_t>(1, std::min<size_t>({(2 * slots + tiles - 1) / tiles,
                                                      steps / (yx::kMmWaves * yx::kMmSteps), 64}));
   if (c->matmul_k_split > 0) ks = std::min<size_t>(static_cast<size_t>(c->matmul_k_split), steps);
-  if (ks > 1 && (rc = matmul_scratch(c, tiles, ks, 256))) return rc;
+  if (ks > 1 && (rc = matmul_scratch(c, tiles, ks))) return rc;
   hipLaunchKernelGGL(yx::matmul_bf16_rows,
                      dim3(static_cast<unsigned>((n + 15) / 16), static_cast<unsigned>((t + 15) / 16),
                           static_cast<unsigned>(ks)),
