@@ -160,3 +160,33 @@ def test_no_alloc_refuses_a_pass_beyond_the_scratch(hip):
                 t.free()
     finally:
         sc.kv.destroy()
+
+
+def test_a_work_list_fits_beside_much_metadata():
+    """A first pass whose page tables nearly fill the smallest staging buffer: the call's work
+    list (five items per sequence and head, three before the chunk search) fits beside them."""
+    from yaxus_amd.backend import HipBackend
+    from yaxus_amd.kv import PassMeta
+
+    hq, hkv, batch, ctx, page = 8, 2, 50, 4475, 16
+    need = -(-(ctx + 1) // page)
+    pages = np.random.default_rng(3).permutation(batch * need).astype(np.uint32)
+    hip = HipBackend(0)
+    try:
+        kv = hip.new_kv(1, batch * need, page, hkv)
+        hip.begin_pass(PassMeta(ids=np.zeros(batch, np.uint32), pos=np.full(batch, ctx, np.uint32),
+                                kv_slot=pages[need - 1::need] * page + ctx % page,
+                                pt_off=np.arange(batch, dtype=np.uint32) * need, pages=pages))
+        rng = np.random.default_rng(4)
+        k, v, q = (hip.tensor(s).upload(rng.standard_normal(s).astype(np.float32))
+                   for s in ((batch, hkv * D), (batch, hkv * D), (batch, hq * D)))
+        scale = float(np.float32(1.0) / np.sqrt(np.float32(D)))
+        outs = []
+        for fn in (hip.L.yx_attention_append_noalloc, hip.L.yx_attention_append_dev):
+            o = hip.tensor((batch, hq * D))
+            check_hip(fn(hip.ctx, kv.h, 0, k.ptr, v.ptr, q.ptr, o.ptr, hq, hkv, 0, scale))
+            outs.append(o.numpy())
+        assert np.array_equal(outs[0], outs[1])
+        kv.destroy()
+    finally:
+        hip.close()

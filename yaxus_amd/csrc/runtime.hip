@@ -115,9 +115,11 @@ struct Staging {
     return YX_OK;
   }
   // Room for `bytes` at the start of an empty staging buffer (grown when needed), to be
-  // filled by the caller and sent with send(): one copy for many pieces.
-  int reserve(size_t bytes, char** out) {
+  // filled by the caller and sent with send(): one copy for many pieces. `more` bytes stay
+  // free behind them for uploads that may not grow it.
+  int reserve(size_t bytes, size_t more, char** out) {
     if (used != 0) return fail(YX_ERR_INVALID, "internal: reserve on a staging buffer in use");
+    bytes += more;
     if (bytes > cap) {
       if (done) YX_HIP(hipEventSynchronize(done));
       if (host) YX_HIP(hipHostFree(host));
@@ -2003,7 +2005,10 @@ int yx_pass_begin(yx_ctx* c, size_t rows, const uint32_t* pos, const uint32_t* k
   const size_t total = std::max<size_t>(off, 256);
   if ((rc = c->d_meta.ensure(total, c->stream))) return rc;
   char* h = nullptr;
-  if ((rc = st.reserve(total, &h))) return rc;
+  // Work lists built after this (for calls the previous pass did not make) find room too
+  // through the entry point that allocates nothing: the chunk searches make a list longer by
+  // up to 7 KiB (12000 sampled passes).
+  if ((rc = st.reserve(total, 64 << 10, &h))) return rc;
   std::memcpy(h + o_pos, pos, rows * 4);
   std::memcpy(h + o_slot, kv_slot, rows * 4);
   if (!runs.empty()) std::memcpy(h + o_runs, runs.data(), runs.size() * 4);
