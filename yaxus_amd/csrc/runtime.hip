@@ -17,6 +17,7 @@
 #include "attn_decode.hpp"
 #include "attn_prefill.hpp"
 #include "attn_prefill_f32.hpp"
+#include "deal.hpp"
 #include "kv_kernels.hpp"
 #include "qk_rope.hpp"
 #include "step_after.hpp"
@@ -662,30 +663,39 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
         if (!sp.pairs || pairs <= sp.over) return 1u;
         return std::max(1u, std::min({(pairs + sp.pairs - 1) / sp.pairs, pairs / std::min(sp.pairs, kMinChunkPairs), 64u}));
       };
-      std::vector<uint32_t> lens, load;
+      // Tiles by their pairs, so that an estimate looks at each length once.
+      std::vector<std::pair<uint32_t, uint32_t>> tiles;  // (pairs, tiles of so many)
+      {
+        std::vector<uint32_t> by_pairs;
+        for (const yx::PrefillItem& w : plan.pitems) {
+          const uint32_t pairs = (w.blk1 - w.blk0 + 1) / 2;
+          if (pairs >= by_pairs.size()) by_pairs.resize(std::max<size_t>(pairs + 1, 2 * by_pairs.size()), 0u);
+          ++by_pairs[pairs];
+        }
+        for (uint32_t pairs = 0; pairs < by_pairs.size(); ++pairs)
+          if (by_pairs[pairs]) tiles.emplace_back(pairs, by_pairs[pairs]);
+      }
+      yx::Deal deal;
+      std::vector<uint32_t> lens;
       size_t parts = 0;       // partial slots of the split last estimated
       double balance = 0;     // and its load per slot
       // At least `cutoff`: the balance alone says so (the deal is left out).
       auto estimate = [&](const Split& sp, double cutoff) {
-        lens.clear();
+        deal.clear();
         parts = 0;
-        uint64_t sum = 0;
-        for (const yx::PrefillItem& w : plan.pitems) {
-          const uint32_t pairs = (w.blk1 - w.blk0 + 1) / 2, nch = chunks(pairs, sp);
-          if (nch > 1) parts += nch;
-          for (uint32_t ch = 0; ch < nch; ++ch) {
-            const uint32_t n = static_cast<uint32_t>(static_cast<uint64_t>(pairs) * (ch + 1) / nch) -
-                               static_cast<uint32_t>(static_cast<uint64_t>(pairs) * ch / nch);
-            lens.push_back(n + kFixedPairs + split_cost(nch));
-            sum += lens.back();
-          }
+        for (const auto& t : tiles) {
+          const uint32_t nch = chunks(t.first, sp), n = t.first / nch, more = t.first % nch;
+          if (nch > 1) parts += static_cast<size_t>(nch) * t.second;
+          const uint32_t own = kFixedPairs + split_cost(nch);  // `more` chunks have a pair more
+          deal.add(n + 1 + own, more * t.second);
+          deal.add(n + own, (nch - more) * t.second);
         }
-        load.assign(std::max<size_t>(1, slots2 / hkv), 0);
-        balance = static_cast<double>(sum) / load.size();
+        const size_t slots = std::max<size_t>(1, slots2 / hkv);
+        balance = static_cast<double>(deal.sum()) / slots;
         if (balance >= cutoff) return balance;
-        std::sort(lens.begin(), lens.end(), std::greater<uint32_t>());
-        if (per_cu == 2 && lens.size() <= load.size()) {
-          const size_t cus = std::max<size_t>(1, load.size() / 2);
+        if (per_cu == 2 && deal.items() <= slots) {
+          deal.sorted(lens);
+          const size_t cus = std::max<size_t>(1, slots / 2);
           double most = 0;
           for (size_t j = 0; j < std::min(cus, lens.size()); ++j) {
             const double beside = j + cus < lens.size() ? lens[j + cus] : 0;
@@ -693,14 +703,8 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
           }
           return most;
         }
-        uint32_t most = 0;
-        for (uint32_t n : lens) {  // a min-heap of the slots' loads
-          std::pop_heap(load.begin(), load.end(), std::greater<uint32_t>());
-          load.back() += n;
-          most = std::max(most, load.back());
-          std::push_heap(load.begin(), load.end(), std::greater<uint32_t>());
-        }
-        return lens.size() > load.size() ? balance + kTail * (most - balance) : most;
+        const uint32_t most = deal.busiest(slots);
+        return deal.items() > slots ? balance + kTail * (most - balance) : most;
       };
       // Partials that fit the scratch of the entry point that allocates nothing keep fitting.
       const size_t part_bytes = hkv * plan.part_rows * (yx::kD * sizeof(float) + sizeof(float2));
@@ -887,8 +891,9 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
   // Bounds of chunk ch of nch of a group of nb blocks: on quads of blocks, or, where a
   // chunk is too long for the queue kernel, on eights (the 16-row-tile kernel's waves
   // then take equal shares of every chunk but the group's last).
+  auto chunk_unit = [](uint32_t nb, uint32_t nch) -> uint32_t { return nb > nch * 4 * yx::kBalQuads ? yx::kWideWaves : 4; };
   auto chunk_begin = [&](uint32_t nb, uint32_t ch, uint32_t nch) {
-    const uint32_t unit = nb > nch * 4 * yx::kBalQuads ? yx::kWideWaves : 4, n = (nb + unit - 1) / unit;
+    const uint32_t unit = chunk_unit(nb, nch), n = (nb + unit - 1) / unit;
     return std::min(nb, unit * static_cast<uint32_t>(static_cast<uint64_t>(n) * ch / nch));
   };
   // Whether every chunk's blocks split evenly over kWideWaves waves.
@@ -936,53 +941,81 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
   // the same L2, counts 0.6; and the new length has to be 13% better. Over 107 sampled
   // passes of 8-48 sequences with a shared prefix 1.11x on average, the slowest 0.978 (dealt
   // longest first, prefixes in full and any gain taken: 1.08x, 17 passes 2-10% slower).
-  std::vector<uint32_t> lens, load;
-  auto estimate = [&](size_t cbk, double cutoff) {
-    constexpr uint32_t kStartBlocks = 16;
-    constexpr double kTail = 0.6;
-    lens.clear();
-    auto add = [&](uint32_t nb, uint32_t tenths) {
-      const uint32_t nq = (nb + 3) / 4, cq = chunk_quads(nq, cbk), nch = (nq + cq - 1) / cq;
-      for (uint32_t ch = 0; ch < nch; ++ch)
-        lens.push_back((chunk_begin(nb, ch + 1, nch) - chunk_begin(nb, ch, nch)) * tenths / 10 + kStartBlocks);
+  yx::Deal deal;
+  const bool in_order = !cascs.empty();
+  // The groups by their blocks (without shared prefixes, those of a length together), with the
+  // fewest quads their chunks have.
+  struct Len {
+    uint32_t nb, groups, least;
+    bool slots;  // partial slots even for one chunk
+  };
+  std::vector<Len> group_lens;
+  auto list_lens = [&]() {
+    auto add = [&](uint32_t nb, uint32_t groups, bool slots) {
+      group_lens.push_back({nb, groups, chunk_quads((nb + 3) / 4, 0), slots});
     };
-    for (const Casc& cc : cascs) add(cc.blocks, 6);
-    for (const Sub& sb : subs) add(sb.b1 - sb.b0, 10);
-    // Slots of one head: the heads' items are alike.
-    load.assign(std::max<size_t>(1, static_cast<size_t>(c->cus) / hkv), 0);
-    uint64_t total = 0;
-    for (uint32_t n : lens) total += n;
-    const double avg = static_cast<double>(total) / load.size();
-    if (avg >= cutoff) return avg;  // no deal is better than the average
-    if (cascs.empty()) std::sort(lens.begin(), lens.end(), std::greater<uint32_t>());
-    uint32_t most = 0;
-    for (uint32_t n : lens) {  // min-heap of the slots' loads
-      std::pop_heap(load.begin(), load.end(), std::greater<uint32_t>());
-      load.back() += n;
-      most = std::max(most, load.back());
-      std::push_heap(load.begin(), load.end(), std::greater<uint32_t>());
+    for (const Casc& cc : cascs) add(cc.blocks, 1, true);
+    if (in_order) {
+      for (const Sub& sb : subs) add(sb.b1 - sb.b0, 1, sb.casc >= 0);
+      return;
     }
-    return avg + kTail * (most - avg);
+    std::vector<uint32_t> by_blocks;
+    for (const Sub& sb : subs) {
+      const uint32_t nb = sb.b1 - sb.b0;
+      if (nb >= by_blocks.size()) by_blocks.resize(std::max<size_t>(nb + 1, 2 * by_blocks.size()), 0u);
+      ++by_blocks[nb];
+    }
+    for (uint32_t nb = 0; nb < by_blocks.size(); ++nb)
+      if (by_blocks[nb]) add(nb, by_blocks[nb], false);
+  };
+  auto chunks_of = [](const Len& l, size_t cbk) -> uint32_t {  // as chunk_quads cuts them
+    const uint32_t nq = (l.nb + 3) / 4, cq = std::max(static_cast<uint32_t>((cbk + 3) / 4), l.least);
+    return (nq + cq - 1) / cq;
+  };
+  constexpr uint32_t kStartBlocks = 16;
+  const size_t head_slots = std::max<size_t>(1, static_cast<size_t>(c->cus) / hkv);
+  auto estimate = [&](size_t cbk, double cutoff) {
+    constexpr double kTail = 0.6;
+    deal.clear();
+    for (size_t i = 0; i < group_lens.size(); ++i) {
+      const Len& l = group_lens[i];
+      const uint32_t nch = chunks_of(l, cbk);
+      const uint32_t unit = chunk_unit(l.nb, nch), n = (l.nb + unit - 1) / unit;
+      if (in_order) {  // the bounds of chunk_begin
+        const uint32_t tenths = i < cascs.size() ? 6 : 10;
+        for (uint32_t ch = 1, from = 0; ch <= nch; ++ch) {
+          const uint32_t to = ch == nch ? l.nb : unit * static_cast<uint32_t>(static_cast<uint64_t>(n) * ch / nch);
+          deal.add_in_order((to - from) * tenths / 10 + kStartBlocks);
+          from = to;
+        }
+        continue;
+      }
+      // In any order: `more` chunks of a unit more, the last one cut at nb.
+      const uint32_t more = n % nch, len = n / nch * unit + kStartBlocks, last = len + (more ? unit : 0) - (n * unit - l.nb);
+      deal.add(last, l.groups);
+      deal.add(len + unit, (more ? more - 1 : 0) * l.groups);
+      deal.add(len, (more ? nch - more : nch - 1) * l.groups);
+    }
+    // Slots of one head: the heads' items are alike.
+    const double avg = static_cast<double>(deal.sum()) / head_slots;
+    if (avg >= cutoff) return avg;  // no deal is better than the average
+    return avg + kTail * (deal.busiest(head_slots) - avg);
   };
   bool sort_items = false;
   if (c->target_waves == 0) {
     // Items of all heads; slots: those of groups in several chunks (a partial slot each).
     auto items_of = [&](size_t cbk, size_t* slots = nullptr) {
       size_t n = 0, sl = 0;
-      for (const Casc& cc : cascs) {
-        const uint32_t nq = (cc.blocks + 3) / 4, cq = chunk_quads(nq, cbk);
-        n += (nq + cq - 1) / cq;
-        sl += (nq + cq - 1) / cq;
-      }
-      for (const Sub& sb : subs) {
-        const uint32_t nq = (sb.b1 - sb.b0 + 3) / 4, cq = chunk_quads(nq, cbk), nch = (nq + cq - 1) / cq;
+      for (const Len& l : group_lens) {
+        const size_t nch = static_cast<size_t>(chunks_of(l, cbk)) * l.groups;
         n += nch;
-        if (nch > 1 || sb.casc >= 0) sl += nch;
+        if (nch > l.groups || l.slots) sl += nch;
       }
       if (slots) *slots = sl * hkv;
       return n * hkv;
     };
     const size_t cus = static_cast<size_t>(c->cus), limit = 64 * waves;
+    list_lens();
     if (items_of(cb) > cus) {
       const size_t avg = (work + cus - 1) / cus;
       // Never more partials or items than the scratch of the entry point that allocates
@@ -996,7 +1029,10 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
       auto consider = [&](size_t cbk) {
         cbk = std::min(std::max<size_t>(cbk, 16), limit);
         size_t sl;
-        if (items_of(cbk, &sl) > max_items || sl > max_slots) return;
+        const size_t n = items_of(cbk, &sl);
+        if (n > max_items || sl > max_slots) return;
+        // As estimate's average, from the count alone.
+        if (!in_order && static_cast<double>(work / hkv + kStartBlocks * (n / hkv)) / head_slots >= margin * best_t) return;
         const double t = estimate(cbk, margin * best_t);
         if (t < margin * best_t) {
           best_t = t;
