@@ -88,3 +88,18 @@ def test_streamed_rows_do_not_depend_on_the_pass(hip):
     for start, rows in [(0, 1), (15, 1), (2, 3), (8, 7)]:
         part = _matmul(hip, x[start:start + rows], w)
         assert np.array_equal(part.view(np.uint32), full[start:start + rows].view(np.uint32)), (start, rows)
+
+
+@pytest.mark.parametrize("t,k,n,rows_kernel", [
+    (256, 512, 512, True), (17, 768, 4096, True), (128, 64, 1536, True), (32, 1024, 6144, True),
+    (20, 1024, 4096, True), (256, 1536, 512, False), (64, 1024, 3072, False), (512, 512, 544, False),
+])
+def test_small_products_keep_the_kernel_that_starts_sooner(hip, t, k, n, rows_kernel):
+    """Just above two 16 x 16 tiles per CU, short sums: LDS tiles take up to 1.55 times as long."""
+    x, w, out = hip.tensor((t, k)), hip.tensor((n, k), np.uint16), hip.tensor((t, n))
+    try:
+        hip.matmul_bf16(x, w, out=out)
+        assert (hip.stat("matmul_kernel") == 1) == rows_kernel
+    finally:
+        for b in (x, w, out):
+            b.free()

@@ -353,6 +353,7 @@ struct yx_ctx {
   // its calls need no earlier one to be captured, and (unlike the buffers counted in
   // buffer_gens) leave captured graphs valid.
   DevBuf mt_part, mt_counters;
+  uint64_t mm_kernel = 0, mm_k_parts = 0;  // what the latest matmul ran (tests)
   // options
   long target_waves = 0;  // 0: one work item per CU
   int cus = 256;
@@ -1515,6 +1516,8 @@ int matmul_scratch(yx_ctx* c, size_t tiles, size_t ks) {
 // 16384 15.0 with 4, 16.7 with 2.
 bool matmul_stream(yx_ctx* c, const float* x, const uint16_t* w, float* out, uint32_t t, uint32_t k, uint32_t n) {
   if (k % 256) return false;
+  c->mm_kernel = 2;
+  c->mm_k_parts = 1;
   const uint32_t tiles = (n + 15) / 16, cus = static_cast<uint32_t>(c->cus);
   uint32_t nb = 1, least = UINT32_MAX;
   for (uint32_t b = 1; b <= static_cast<uint32_t>(yx::kStreamMaxBatch); b *= 2) {
@@ -1556,6 +1559,18 @@ int matmul_tiles_scratch(yx_ctx* c) {
   return c->mt_counters.ensure(slots * 4 * yx::kCounterStride, c->stream, true);
 }
 
+// Whether matmul_bf16_rows is the faster kernel for more than 16 rows, from two of its
+// workgroups per CU on: few of them and short sums, which it starts sooner (t x k x n, tiles /
+// rows kernel in us: 256 x 512 x 512 8.6 / 5.7, 17 x 768 x 4096 9.6 / 6.4, 256 x 768 x 768 10.1 /
+// 9.1; up to 32 rows a little further, 17 x 1024 x 6144 11.3 / 10.1; beyond, 64 x 1024 x 3072
+// 9.6 / 10.8, 48 x 1536 x 4096 11.0 / 16.1). Over 1060 shapes of 512-3000 tiles of 16 x 16, k
+// 64-4096, the choice is within 3% of the faster kernel in 1051, 9% at most.
+bool matmul_rows_faster(uint32_t t, uint32_t k, size_t per_cu) {
+  const bool few = t <= 32;
+  const size_t most = k <= 768 ? (few && k > 256 ? 4 : 3) : k <= 1024 ? (few ? 3 : 2) : k <= 1280 ? 2 : 0;
+  return per_cu <= most;
+}
+
 // Many rows: LDS tiles. The tile shape and the split of k with the smallest estimated
 // time: rounds of workgroups times a workgroup's time, its stages of 32 k times the
 // shape's cost per stage (all CUs busy, measured over t 20-4096, k 1536-3072, n
@@ -1588,6 +1603,8 @@ int matmul_tiled(yx_ctx* c, const float* x, const uint16_t* w, float* out, uint3
     }
   }
   const MatmulShape& sh = kMatmulShapes[best];
+  c->mm_kernel = 3 + static_cast<uint64_t>(best);
+  c->mm_k_parts = best_ks;
   const size_t tiles = static_cast<size_t>((t + sh.tm - 1) / sh.tm) * ((n + sh.tn - 1) / sh.tn);
   if (tiles > 0x7fffffff) return fail(YX_ERR_UNSUPPORTED, "matmul dimensions too large");
   const auto go = [&](auto* kern) {
@@ -2083,6 +2100,10 @@ int yx_ctx_get_stat(yx_ctx* c, const char* key, uint64_t* out) {
     *out = c->split_tiles;
   else if (!std::strcmp(key, "prefill_plans"))
     *out = c->prefill_plans;
+  else if (!std::strcmp(key, "matmul_kernel"))
+    *out = c->mm_kernel;
+  else if (!std::strcmp(key, "matmul_k_parts"))
+    *out = c->mm_k_parts;
   else
     return fail(YX_ERR_INVALID, std::string("unknown statistic ") + key);
   return YX_OK;
@@ -2319,7 +2340,8 @@ int yx_matmul_bf16_dev(yx_ctx* c, const float* x, const uint16_t* w, float* out,
         YX_HIP(hipGetLastError());
         return YX_OK;
       }
-    } else if (k <= (size_t{1} << 20)) {  // a tile's rows within a buffer resource
+    } else if (k <= (size_t{1} << 20) &&  // a tile's rows within a buffer resource
+               !matmul_rows_faster(T, K, (tiles16 + slots - 1) / slots)) {
       return matmul_tiled(c, x, w, out, T, K, N);
     }
   }
@@ -2329,6 +2351,8 @@ int yx_matmul_bf16_dev(yx_ctx* c, const float* x, const uint16_t* w, float* out,
   size_t ks = std::max<size_t>(1, std::min<size_t>({(2 * slots + tiles - 1) / tiles,
                                                      steps / (yx::kMmWaves * yx::kMmSteps), 64}));
   if (c->matmul_k_split > 0) ks = std::min<size_t>(static_cast<size_t>(c->matmul_k_split), steps);
+  c->mm_kernel = 1;
+  c->mm_k_parts = ks;
   if (ks > 1 && (rc = matmul_scratch(c, tiles, ks))) return rc;
   hipLaunchKernelGGL(yx::matmul_bf16_rows,
                      dim3(static_cast<unsigned>((n + 15) / 16), static_cast<unsigned>((t + 15) / 16),
