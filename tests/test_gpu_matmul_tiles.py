@@ -1,7 +1,9 @@
 """yx_matmul_bf16_dev beyond one row tile: passes of many rows (LDS tiles of 128 x 256, 128 x
-128, 64 x 128 and 64 x 64, some split along k) and few rows against many weight rows (the
+128, 64 x 128 and 64 x 64, whole and split along k) and few rows against many weight rows (the
 streaming kernel), at the edges of tiles, stages and splits, against the CPU backend's
-restatement (crates/yaxus-backend-cpu/src/lib.rs:234-248, 314-345)."""
+restatement (crates/yaxus-backend-cpu/src/lib.rs:234-248, 314-345) and 64 bits. Each case
+names the kernel and the split that the automatic choice takes on 256 CUs, so that a retuned
+choice cannot drop one unseen."""
 
 import numpy as np
 import pytest
@@ -39,28 +41,61 @@ def _bound(x, w):
     return 2 * x.shape[1] * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(wf).astype(np.float64).T)
 
 
-@pytest.mark.parametrize("t,k,n", [
-    (33, 72, 2728),      # 64 x 64, k no multiple of a stage, an odd number of stages
-    (100, 8, 1300),      # one stage of 8 k
-    (515, 520, 516),     # 64 x 64 split along k, partial tiles on both sides
-    (17, 512, 5000),     # fewer rows than a tile, more weight rows than rows
-    (700, 1032, 1500),   # split along k with a tail
-    (1100, 96, 1030),    # 64 x 128, n even but no multiple of 4 (narrow stores)
-    (64, 2048, 4100),    # 64 x 128 split
-    (1030, 264, 4099),   # 128-row tiles, n odd
-    (2049, 40, 2050),
-    (16, 1024, 8192), (1, 2048, 8200), (7, 1536, 8209), (16, 2560, 16400), (3, 2048, 33000),  # streaming
-    (5, 3072, 8300), (9, 264, 9000),  # few rows, k the streaming kernel is not built for
+ROWS, STREAM, T128x256, T128x128, T64x128, T64x64 = range(1, 7)  # yx_ctx_get_stat's matmul_kernel
+
+
+@pytest.mark.parametrize("t,k,n,kernel,parts", [
+    (33, 72, 2728, ROWS, 1),
+    (100, 8, 1300, ROWS, 1),
+    (45, 72, 5211, T64x64, 1),       # k no multiple of a stage, an odd number of stages, n odd
+    (200, 8, 2100, T64x64, 1),       # one stage of 8 k
+    (515, 520, 516, T64x64, 2),      # partial tiles on both sides
+    (33, 1096, 4333, T64x64, 4),
+    (499, 2056, 249, T64x64, 8),
+    (1100, 96, 1030, T64x128, 1),    # n even but no multiple of 4 (narrow stores)
+    (700, 1032, 1500, T64x128, 1),   # a k tail
+    (21, 712, 8235, T64x128, 2),
+    (64, 2048, 4100, T64x128, 4),
+    (60, 8200, 2100, T64x128, 8),
+    (17, 512, 5000, ROWS, 1),        # fewer rows than a tile, more weight rows than rows
+    (300, 72, 8369, T128x128, 1),
+    (601, 2056, 2047, T128x128, 2),
+    (77, 3352, 4191, T128x128, 4),
+    (1030, 264, 4099, T128x256, 1),
+    (2049, 40, 2050, T128x256, 1),
+    (1029, 2056, 2050, T128x256, 2),
+    (71, 3672, 8230, T128x256, 4),
+    (16, 1024, 8192, STREAM, 1), (1, 2048, 8200, STREAM, 1), (7, 1536, 8209, STREAM, 1),
+    (16, 2560, 16400, STREAM, 1), (3, 2048, 33000, STREAM, 1),
+    (5, 3072, 8300, ROWS, 1), (9, 264, 9000, ROWS, 1),  # k the streaming kernel is not built for
 ])
-def test_matmul_matches_the_cpu_backend(hip, t, k, n):
+def test_matmul_matches_the_cpu_backend(hip, t, k, n, kernel, parts):
     x = normal(t * k, 31, t * 7 + n).reshape(t, k)
     w = _bf16_bits(normal(n * k, 32, k + n).reshape(n, k))
     got = _matmul(hip, x, w)
-    assert np.all(np.abs(got.astype(np.float64) - matmul_bf16(x, w)) <= _bound(x, w))
+    assert (hip.stat("matmul_kernel"), hip.stat("matmul_k_parts")) == (kernel, parts)
+    bound = _bound(x, w)
+    some = np.unique(np.linspace(0, t - 1, 48).astype(int))  # the oracle takes a second per 1.3e9 products
+    assert np.all(np.abs(got[some].astype(np.float64) - matmul_bf16(x[some], w)) <= bound[some])
+    # Against 64 bits: f32 sums are 0.4e-7 to 3.6e-7 off here, x without its third part 1e-5.
+    exact = x.astype(np.float64) @ (w.astype(np.uint32) << 16).view(np.float32).astype(np.float64).T
+    assert np.all(np.abs(got - exact) <= bound)
+    assert np.linalg.norm(got - exact) < 5e-7 * np.linalg.norm(exact)
+    if kernel == STREAM:  # the bits of the kernel of 16 x 16 tiles without a split of k
+        try:
+            hip.set_option("matmul_k_split", 1)
+            rows = _matmul(hip, x, w)
+        finally:
+            hip.set_option("matmul_k_split", 0)
+        assert hip.stat("matmul_kernel") == ROWS
+        assert np.array_equal(got.view(np.uint32), rows.view(np.uint32))
 
 
-@pytest.mark.parametrize("t,k,n", [(130, 264, 2000), (4, 1024, 8192)])
-def test_matmul_carries_infinities_and_nan(hip, t, k, n):
+@pytest.mark.parametrize("t,k,n,kernel,parts", [
+    (130, 264, 2000, T64x64, 1), (4, 1024, 8192, STREAM, 1), (601, 2056, 2047, T128x128, 2),
+    (1029, 2056, 2050, T128x256, 2), (21, 712, 8235, T64x128, 2),
+])
+def test_matmul_carries_infinities_and_nan(hip, t, k, n, kernel, parts):
     """One infinite and one NaN activation: the row's outputs are what the CPU gives
     (infinities of the weight's sign, NaN), the other rows' stay finite and right; values
     near FLT_MAX, whose rounded-up bf16 part would be infinite, stay finite."""
@@ -71,12 +106,16 @@ def test_matmul_carries_infinities_and_nan(hip, t, k, n):
     x[2, 5] = np.inf
     x[t - 1, 3] = np.nan
     got = _matmul(hip, x, w)
+    assert (hip.stat("matmul_kernel"), hip.stat("matmul_k_parts")) == (kernel, parts)
+    some = [0, 1, 2, *range(3, t - 1, 1 + t // 48), t - 1]
     with np.errstate(over="ignore", invalid="ignore"):
-        want = matmul_bf16(x, w)
-    fine = [i for i in range(t) if i not in (2, t - 1)]
+        want = dict(zip(some, matmul_bf16(x[some], w)))
     assert np.array_equal(got[2], want[2]) and np.isinf(got[2]).all()
     assert np.isnan(got[t - 1]).all()
-    assert np.all(np.abs(got[fine].astype(np.float64) - want[fine]) <= _bound(x[fine], w))
+    assert np.isfinite(np.delete(got, (2, t - 1), 0)).all()
+    for i in some:
+        if i not in (2, t - 1):
+            assert np.all(np.abs(got[i].astype(np.float64) - want[i]) <= _bound(x[i:i + 1], w)[0])
 
 
 def test_streamed_rows_do_not_depend_on_the_pass(hip):
