@@ -100,9 +100,9 @@ __global__ __launch_bounds__(kMatmulThreads, T::kWavesPerSimd) void matmul_bf16_
   constexpr int TM = T::TM, TN = T::TN, KU = T::KU, KT = T::KT, TH = kMatmulThreads;
   static_assert(T::WM * T::WN * 64 == TH, "8 waves");
   constexpr int MT = TM / T::WM / 16, NT = TN / T::WN / 16;  // 16 x 16 tiles per wave
-  // Chunks of 8 k per stage, and per thread (the last round may be partial).
-  constexpr int kXChunks = TM * KT / 8, kWChunks = TN * KT / 8;
-  constexpr int XC = (kXChunks + TH - 1) / TH, WC = (kWChunks + TH - 1) / TH;
+  // Chunks of 8 k per thread and stage.
+  constexpr int XC = TM * KT / 8 / TH, WC = TN * KT / 8 / TH;
+  static_assert(TM * KT / 8 == XC * TH && TN * KT / 8 == WC * TH, "whole rounds of chunks");
   constexpr int kOutside = 0x7ffffff0;  // beyond every resource: reads zeros
   __shared__ u16x8 xs[2][KU][3][TM * 4];
   __shared__ u16x8 ws[2][KU][TN * 4];
@@ -123,8 +123,6 @@ __global__ __launch_bounds__(kMatmulThreads, T::kWavesPerSimd) void matmul_bf16_
   const uint32_t s1 = static_cast<uint32_t>(static_cast<uint64_t>(stages) * (kp + 1) / ks);
   const uint32_t seg = max(2u, (stages >> 3) & ~1u);  // stages per partial sum (even: the slots alternate)
 
-  const auto has_x = [&](int i) { return (i + 1) * TH <= kXChunks || i * TH + tid < kXChunks; };
-  const auto has_w = [&](int i) { return (i + 1) * TH <= kWChunks || i * TH + tid < kWChunks; };
   int xd[XC], wd[WC], xo[XC], wo[WC];  // LDS chunk, global byte offset in the tile's rows
   uint32_t xk[XC], wk[WC];             // first k of the chunk within its stage
 #pragma unroll
@@ -160,7 +158,6 @@ __global__ __launch_bounds__(kMatmulThreads, T::kWavesPerSimd) void matmul_bf16_
     const bool tail = kb + KT > k;  // uniform
 #pragma unroll
     for (int i = 0; i < XC; ++i) {
-      if (!has_x(i)) continue;
       const int o = tail && kb + xk[i] >= k ? kOutside : xo[i];
       r.a[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, o, kb * 4, 0));
       r.b[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, o, kb * 4 + 16, 0));
@@ -171,7 +168,6 @@ __global__ __launch_bounds__(kMatmulThreads, T::kWavesPerSimd) void matmul_bf16_
     const bool tail = kb + KT > k;
 #pragma unroll
     for (int i = 0; i < WC; ++i) {
-      if (!has_w(i)) continue;
       const int o = tail && kb + wk[i] >= k ? kOutside : wo[i];
       r.v[i] = __builtin_bit_cast(u16x8, __builtin_amdgcn_raw_buffer_load_b128(rw, o, kb * 2, 0));
     }
@@ -202,13 +198,11 @@ __global__ __launch_bounds__(kMatmulThreads, T::kWavesPerSimd) void matmul_bf16_
     u16x8* wb = &ws[slot][0][0];
 #pragma unroll
     for (int i = 0; i < XC; ++i) {
-      if (!has_x(i)) continue;
 #pragma unroll
       for (int q = 0; q < 3; ++q) xb[xd[i] + q * TM * 4] = __builtin_bit_cast(u16x8, xp.p[i][q]);
     }
 #pragma unroll
-    for (int i = 0; i < WC; ++i)
-      if (has_w(i)) wb[wd[i]] = wr.v[i];
+    for (int i = 0; i < WC; ++i) wb[wd[i]] = wr.v[i];
   };
   bf16x8 wf[KU][NT], xf[KU][MT][3];
   const auto read_operands = [&](int slot) {
@@ -238,13 +232,10 @@ __global__ __launch_bounds__(kMatmulThreads, T::kWavesPerSimd) void matmul_bf16_
                 wf[u][a], xf[u][b][q], decltype(first)::value && u == 0 && q == 0 ? f32x4{0, 0, 0, 0} : acc[a][b],
                 0, 0, 0);
   };
-  // A workgroup barrier that orders LDS accesses only: global loads stay in flight.
-  const auto barrier = [&]() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  const auto barrier = []() {  // nothing moves from one phase to the other
     __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_barrier();
+    lds_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
   };
   // Every wave passes the same number of barriers: the late group one more before its
   // first stage, the other one more after its last. Stage s + 1 is in its slot once both
@@ -431,10 +422,7 @@ __global__ __launch_bounds__(64 * kStreamWaves, 2) void matmul_bf16_stream(
           acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wv[d][u]), xf[u][q], acc, 0, 0, 0);
       part[half][j][wave][lane] = acc;
       if (++j < nb) continue;
-      // LDS only: the next tile's loads stay in flight.
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-      __builtin_amdgcn_s_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+      lds_barrier();  // the next tile's loads stay in flight
       const uint32_t tile = b * nb + wave;
       if (static_cast<uint32_t>(wave) < nb && tile < tiles) {
         f32x4 s = part[half][wave][0][lane];
