@@ -47,14 +47,14 @@ ROWS, STREAM, T128x256, T128x128, T64x128, T64x64 = range(1, 7)  # yx_ctx_get_st
 @pytest.mark.parametrize("t,k,n,kernel,parts", [
     (33, 72, 2728, ROWS, 1),
     (100, 8, 1300, ROWS, 1),
-    (45, 72, 5211, T64x64, 1),       # k no multiple of a stage, an odd number of stages, n odd
+    (45, 72, 9211, T64x64, 1),       # k no multiple of a stage, an odd number of stages, n odd
     (200, 8, 2100, T64x64, 1),       # one stage of 8 k
     (515, 520, 516, T64x64, 2),      # partial tiles on both sides
     (33, 1096, 4333, T64x64, 4),
     (499, 2056, 249, T64x64, 8),
     (1100, 96, 1030, T64x128, 1),    # n even but no multiple of 4 (narrow stores)
     (700, 1032, 1500, T64x128, 1),   # a k tail
-    (21, 712, 8235, T64x128, 2),
+    (21, 1288, 8235, T64x128, 2),
     (64, 2048, 4100, T64x128, 4),
     (60, 8200, 2100, T64x128, 8),
     (17, 512, 5000, ROWS, 1),        # fewer rows than a tile, more weight rows than rows
@@ -92,8 +92,8 @@ def test_matmul_matches_the_cpu_backend(hip, t, k, n, kernel, parts):
 
 
 @pytest.mark.parametrize("t,k,n,kernel,parts", [
-    (130, 264, 2000, T64x64, 1), (4, 1024, 8192, STREAM, 1), (601, 2056, 2047, T128x128, 2),
-    (1029, 2056, 2050, T128x256, 2), (21, 712, 8235, T64x128, 2),
+    (130, 264, 4000, T64x64, 1), (4, 1024, 8192, STREAM, 1), (601, 2056, 2047, T128x128, 2),
+    (1029, 2056, 2050, T128x256, 2), (21, 1288, 8235, T64x128, 2),
 ])
 def test_matmul_carries_infinities_and_nan(hip, t, k, n, kernel, parts):
     """One infinite and one NaN activation: the row's outputs are what the CPU gives
@@ -132,6 +132,8 @@ def test_streamed_rows_do_not_depend_on_the_pass(hip):
 @pytest.mark.parametrize("t,k,n,rows_kernel", [
     (256, 512, 512, True), (17, 768, 4096, True), (128, 64, 1536, True), (32, 1024, 6144, True),
     (20, 1024, 4096, True), (256, 1536, 512, False), (64, 1024, 3072, False), (512, 512, 544, False),
+    (603, 408, 387, True), (112, 952, 1210, True), (1826, 408, 102, True), (232, 624, 923, True),
+    (259, 968, 600, True), (1964, 968, 112, False), (3000, 1000, 144, False),
 ])
 def test_small_products_keep_the_kernel_that_starts_sooner(hip, t, k, n, rows_kernel):
     """Just above two 16 x 16 tiles per CU, short sums: LDS tiles take up to 1.55 times as long."""

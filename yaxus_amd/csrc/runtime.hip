@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <map>
@@ -1559,18 +1560,6 @@ int matmul_tiles_scratch(yx_ctx* c) {
   return c->mt_counters.ensure(slots * 4 * yx::kCounterStride, c->stream, true);
 }
 
-// Whether matmul_bf16_rows is the faster kernel for more than 16 rows, from two of its
-// workgroups per CU on: few of them and short sums, which it starts sooner (t x k x n, tiles /
-// rows kernel in us: 256 x 512 x 512 8.6 / 5.7, 17 x 768 x 4096 9.6 / 6.4, 256 x 768 x 768 10.1 /
-// 9.1; up to 32 rows a little further, 17 x 1024 x 6144 11.3 / 10.1; beyond, 64 x 1024 x 3072
-// 9.6 / 10.8, 48 x 1536 x 4096 11.0 / 16.1). Over 1060 shapes of 512-3000 tiles of 16 x 16, k
-// 64-4096, the choice is within 3% of the faster kernel in 1051, 9% at most.
-bool matmul_rows_faster(uint32_t t, uint32_t k, size_t per_cu) {
-  const bool few = t <= 32;
-  const size_t most = k <= 768 ? (few && k > 256 ? 4 : 3) : k <= 1024 ? (few ? 3 : 2) : k <= 1280 ? 2 : 0;
-  return per_cu <= most;
-}
-
 // Many rows: LDS tiles. The tile shape and the split of k with the smallest estimated
 // time: rounds of workgroups times a workgroup's time, its stages of 32 k times the
 // shape's cost per stage (all CUs busy, measured over t 20-4096, k 1536-3072, n
@@ -1579,11 +1568,14 @@ bool matmul_rows_faster(uint32_t t, uint32_t k, size_t per_cu) {
 // the fastest or one within 5% of it in those shapes (t 4096, n 2048: 128 x 256 tiles 87
 // us, 128 x 128 114, 64 x 128 123; t 512: 64 x 128 split in two 22.3, 128 x 128 in four
 // 22.9, 128 x 256 in two 45; t 80: 64 x 64 in four 12.0, 64 x 128 in eight 12.7).
-int matmul_tiled(yx_ctx* c, const float* x, const uint16_t* w, float* out, uint32_t t, uint32_t k, uint32_t n) {
+struct MatmulSplit {
+  int shape;
+  uint32_t ks;
+  double us;  // estimated
+};
+MatmulSplit matmul_tile_split(yx_ctx* c, uint32_t t, uint32_t k, uint32_t n) {
   const uint32_t steps = (k + 31) / 32;
-  int best = 0;
-  uint32_t best_ks = 1;
-  double best_us = 1e30;
+  MatmulSplit best{0, 1, 1e30};
   for (int s = 0; s < 4; ++s) {
     const MatmulShape& sh = kMatmulShapes[s];
     const uint64_t tiles = static_cast<uint64_t>((t + sh.tm - 1) / sh.tm) * ((n + sh.tn - 1) / sh.tn);
@@ -1593,26 +1585,45 @@ int matmul_tiled(yx_ctx* c, const float* x, const uint16_t* w, float* out, uint3
       // A CU with one workgroup where two fit runs it faster.
       const double stage = tiles * ks * sh.per_cu <= slots ? sh.stage_us * 0.6 : sh.stage_us;
       const double one = sh.per_cu == 1 ? sh.stage_us : stage;
-      const double us = 5.0 + rounds * (one * steps / ks + 1.0) + 
+      const double us = 5.0 + rounds * (one * steps / ks + 1.0) +
                         (ks > 1 ? 1.0 + ks * (sh.tm * sh.tn) / 12500.0 : 0.0);
-      if (us < best_us) {
-        best_us = us;
-        best = s;
-        best_ks = ks;
-      }
+      if (us < best.us) best = {s, ks, us};
     }
   }
-  const MatmulShape& sh = kMatmulShapes[best];
-  c->mm_kernel = 3 + static_cast<uint64_t>(best);
-  c->mm_k_parts = best_ks;
+  return best;
+}
+
+// Whether matmul_bf16_rows is the faster kernel for more than 16 rows, from two of its
+// workgroups per CU on: few of them and short sums, which it starts sooner. Its time in us by
+// least squares over 2500 shapes (512-16000 tiles of 16 x 16, t 17-8000, k 64-2400, n 16-12000,
+// no two sizes alike): its start, per workgroup of a CU the 32-wide steps of k and the passes of
+// its loop, and x's reads by up to 8 XCDs; the tiles' estimate, with their narrower stores where n
+// is no multiple of 4. (t x k x n, tiles / rows kernel in us: 603 x 408 x 387 10.2 / 7.2, 112 x
+// 952 x 1210 12.1 / 8.7, 256 x 512 x 512 8.6 / 5.7, 17 x 768 x 4096 9.6 / 6.4; on the other side
+// 1964 x 968 x 112 11.7 / 21.3, 64 x 1024 x 3072 9.6 / 10.8.) The faster kernel, or one within 4%
+// of it, in 2412 of them; by k and workgroups per CU alone 2212, 58% at most. From k about 1280 on
+// tiles are never more than 6% slower.
+bool matmul_rows_faster(yx_ctx* c, uint32_t t, uint32_t k, uint32_t n, double tiles_us) {
+  if (k > 1280) return false;
+  const double nt = (n + 15) / 16, per_cu = nt * ((t + 15) / 16) / c->cus, steps = (k + 31) / 32;
+  const double passes = std::ceil(steps / (yx::kMmWaves * yx::kMmSteps)), x_mb = 4e-6 * t * k;
+  const double rows_us = 2.65 + per_cu * (steps / 16 - 0.5) + std::ceil(per_cu) * passes + 0.043 * x_mb * std::min(8.0, nt);
+  return rows_us < 1.05 * tiles_us - 1.5 + (n % 4 ? 0.9 : 0.0);
+}
+
+int matmul_tiled(yx_ctx* c, const float* x, const uint16_t* w, float* out, uint32_t t, uint32_t k, uint32_t n,
+                 const MatmulSplit& split) {
+  const MatmulShape& sh = kMatmulShapes[split.shape];
+  c->mm_kernel = 3 + static_cast<uint64_t>(split.shape);
+  c->mm_k_parts = split.ks;
   const size_t tiles = static_cast<size_t>((t + sh.tm - 1) / sh.tm) * ((n + sh.tn - 1) / sh.tn);
   if (tiles > 0x7fffffff) return fail(YX_ERR_UNSUPPORTED, "matmul dimensions too large");
   const auto go = [&](auto* kern) {
-    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(tiles), best_ks), dim3(yx::kMatmulThreads), 0, c->stream, x,
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(tiles), split.ks), dim3(yx::kMatmulThreads), 0, c->stream, x,
                        w, out, t, k, n, static_cast<yx::f32x4*>(c->mt_part.p),
                        static_cast<uint32_t>(c->mt_part.cap), static_cast<uint32_t*>(c->mt_counters.p));
   };
-  switch (best) {
+  switch (split.shape) {
     case 0: go(yx::matmul_bf16_tiles<yx::MatmulTileA>); break;
     case 1: go(yx::matmul_bf16_tiles<yx::MatmulTileB>); break;
     case 2: go(yx::matmul_bf16_tiles<yx::MatmulTileC>); break;
@@ -2340,9 +2351,9 @@ int yx_matmul_bf16_dev(yx_ctx* c, const float* x, const uint16_t* w, float* out,
         YX_HIP(hipGetLastError());
         return YX_OK;
       }
-    } else if (k <= (size_t{1} << 20) &&  // a tile's rows within a buffer resource
-               !matmul_rows_faster(T, K, (tiles16 + slots - 1) / slots)) {
-      return matmul_tiled(c, x, w, out, T, K, N);
+    } else if (k <= (size_t{1} << 20)) {  // a tile's rows within a buffer resource
+      const MatmulSplit split = matmul_tile_split(c, T, K, N);
+      if (!matmul_rows_faster(c, T, K, N, split.us)) return matmul_tiled(c, x, w, out, T, K, N, split);
     }
   }
   // Workgroups per output tile along k: about two workgroups per CU in all, each wave
