@@ -87,7 +87,8 @@ int yx_ctx_set_option(yx_ctx* ctx, const char* key, long value);
 /* Counters of the context since its creation: "page_entries_sent" (page-table entries
  * yx_pass_begin uploaded), "page_runs_sent" (runs of consecutive entries they formed)
  * "prefill_split_tiles" (prefill tiles split along keys in the work lists built) and
- * "prefill_plans" (work lists built as prefill tiles rather than decode items). And of its
+ * "prefill_plans" (work lists built as prefill tiles rather than decode items); "decode_items",
+ * the items, of all heads, of the latest list of decode items. And of its
  * latest yx_matmul_bf16_dev: "matmul_kernel" (0 none yet, 1 the kernel of 16 x 16 tiles, 2 the
  * one that streams the weight, 3 to 6 LDS tiles of 128 x 256, 128 x 128, 64 x 128, 64 x 64) and
  * "matmul_k_parts" (the workgroups of a tile along k).

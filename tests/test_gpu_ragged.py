@@ -5,6 +5,8 @@ item in turn), against the oracle and against a split forced by an option."""
 import numpy as np
 import pytest
 
+from yaxus_amd.kv import PassMeta
+
 from tests.scenario import D, Scenario, close
 
 pytestmark = pytest.mark.gpu
@@ -77,3 +79,36 @@ def test_prefill_chunks_of_long_tiles(hip, chunks, priors, hq, hkv, window, f32)
     finally:
         hip.set_option("prefill_split", 1)
         sc.kv.destroy()
+
+
+def _forks(batch, rows, ctx, prefix, page):
+    """The metadata of `rows` rows for each of `batch` sequences after ctx keys, the first
+    `prefix` of them on shared pages: (pool pages, pass)."""
+    shared, own = prefix // page, -(-(ctx + rows) // page) - prefix // page
+    tables = [np.r_[0:shared, shared + i * own:shared + (i + 1) * own].astype(np.uint32) for i in range(batch)]
+    p = np.arange(ctx, ctx + rows, dtype=np.uint32)
+    return shared + batch * own, PassMeta(
+        ids=np.zeros(batch * rows, np.uint32), pos=np.tile(p, batch),
+        kv_slot=np.concatenate([t[p // page] * np.uint32(page) + p % page for t in tables]),
+        pt_off=np.repeat(np.arange(batch, dtype=np.uint32) * len(tables[0]), rows), pages=np.concatenate(tables))
+
+
+@pytest.mark.parametrize("batch,rows,ctx,prefix,hq,hkv,f32,items", [
+    (74, 7, 1250, 0, 16, 4, False, 296),       # shorter chunks estimated 1% better, 14% slower
+    (134, 1, 1230, 0, 14, 2, False, 268),      # a few items beyond one round
+    (22, 2, 2461, 2432, 40, 8, True, 352),     # f32 forks that read each other's pages
+])
+def test_work_lists_stay_whole_where_a_cut_does_not_pay(hip, batch, rows, ctx, prefix, hq, hkv, f32, items):
+    """Passes that a longer or shorter chunk length made slower keep the plain split's items."""
+    pool, meta = _forks(batch, rows, ctx, prefix, 32)
+    kv = hip.new_kv(1, pool, 32, hkv, D, f32=f32)
+    try:
+        hip.begin_pass(meta)
+        split0 = hip.stat("prefill_split_tiles")
+        hip.attend(kv, 0, np.zeros((batch * rows, hq * D), np.float32), hq)
+        if items is None:
+            assert hip.stat("prefill_split_tiles") == split0
+        else:
+            assert hip.stat("decode_items") == items
+    finally:
+        kv.destroy()

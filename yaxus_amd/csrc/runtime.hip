@@ -323,6 +323,7 @@ struct yx_ctx {
   std::vector<std::tuple<size_t, size_t, size_t, bool, size_t>> used_keys;  // plans used this pass
   uint64_t pages_sent = 0, runs_sent = 0;        // page-table entries and runs uploaded (tests)
   uint64_t split_tiles = 0;                       // prefill tiles split along keys (tests)
+  uint64_t decode_items = 0;                      // items, of all heads, of the latest list of decode items (tests)
   uint64_t prefill_plans = 0;                     // work lists built as prefill tiles (tests)
   bool have_pass = false;
   std::map<std::tuple<size_t, size_t, size_t, bool, size_t>, AttnPlan> plans;  // (window, hq, hkv, f32, page)
@@ -941,8 +942,8 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
   // 102.8 -> 78.8. With shared prefixes the items keep their order (their XCD placement),
   // so the estimate deals them in it; a block of a prefix, which its other groups read from
   // the same L2, counts 0.6; and the new length has to be 13% better. Over 107 sampled
-  // passes of 8-48 sequences with a shared prefix 1.11x on average, the slowest 0.978 (dealt
-  // longest first, prefixes in full and any gain taken: 1.08x, 17 passes 2-10% slower).
+  // passes of 8-48 sequences with a shared prefix, binary16, 1.11x on average, the slowest 0.978
+  // (dealt longest first, prefixes in full and any gain taken: 1.08x, 17 passes 2-10% slower).
   yx::Deal deal;
   const bool in_order = !cascs.empty();
   // The groups by their blocks (without shared prefixes, those of a length together), with the
@@ -1018,6 +1019,12 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
     };
     const size_t cus = static_cast<size_t>(c->cus), limit = 64 * waves;
     list_lens();
+    // Forks beside each other in the pass, without a shared prefix of their own above: they read
+    // the same pages.
+    bool forks = false;
+    for (size_t i = 1; i < subs.size() && !in_order && !forks; ++i)
+      forks = subs[i].dev_off != subs[i - 1].dev_off && std::max(subs[i].pt_off, subs[i - 1].pt_off) < c->pages.size() &&
+              c->pages[subs[i].pt_off] == c->pages[subs[i - 1].pt_off];
     if (items_of(cb) > cus) {
       const size_t avg = (work + cus - 1) / cus;
       // Never more partials or items than the scratch of the entry point that allocates
@@ -1026,17 +1033,22 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
       const size_t items0 = items_of(cb, &slots0);
       const size_t max_slots = std::max<size_t>(slots0, 640), max_items = std::max<size_t>(items0, 8192);
       size_t best = cb;
-      double best_t = estimate(cb, 1e30);
+      const double plain_t = estimate(cb, 1e30);
+      double best_t = plain_t;
       const double margin = cascs.empty() ? 1.0 : 0.87;
-      auto consider = [&](size_t cbk) {
+      // Forks' items read each other's pages from cache while they run side by side: no fewer
+      // than 0.6 of them (f32, 2 and 4 rows, 464 -> 232 items 113 -> 127 us, 352 -> 176 86 -> 92).
+      const size_t least_items = forks ? items0 * 6 / 10 : 0;
+      auto consider = [&](size_t cbk, double of_plain) {
         cbk = std::min(std::max<size_t>(cbk, 16), limit);
+        const double below = std::min(margin * best_t, of_plain * plain_t);
         size_t sl;
         const size_t n = items_of(cbk, &sl);
-        if (n > max_items || sl > max_slots) return;
+        if (n > max_items || n < least_items || sl > max_slots) return;
         // As estimate's average, from the count alone.
-        if (!in_order && static_cast<double>(work / hkv + kStartBlocks * (n / hkv)) / head_slots >= margin * best_t) return;
-        const double t = estimate(cbk, margin * best_t);
-        if (t < margin * best_t) {
+        if (!in_order && static_cast<double>(work / hkv + kStartBlocks * (n / hkv)) / head_slots >= below) return;
+        const double t = estimate(cbk, below);
+        if (t < below) {
           best_t = t;
           best = cbk;
         }
@@ -1047,11 +1059,21 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
           const size_t mid = (lo + hi) / 2;
           (items_of(mid) > cus ? lo : hi) = mid;
         }
-        consider(hi);
+        consider(hi, 1.0);
       }
-      for (size_t p : {60, 80, 100, 115, 135, 160}) consider(avg * p / 100);
+      // Shorter chunks than the plain split's cost starts and merges that the estimate is not
+      // exact enough for: at least 3% better (74 x 7 rows after 1124-1378 keys, 1% estimated: 60 ->
+      // 68 us), and 10% where the plain split of a binary16 pass has few items more than CUs, which
+      // run alone at the end (134 sequences of 1230 keys, 2 KV heads, 268 items: 40.8 -> 43.5 us). Many
+      // rounds over an f32 arena's shared prefixes are even already (864 -> 648 items 77 -> 88 us).
+      if (!(f32 && in_order && items0 >= 3 * cus))
+        for (size_t p : {60, 80, 100, 115, 135, 160})
+          consider(avg * p / 100, avg * p / 100 >= cb ? 1.0 : !f32 && 5 * items0 < 6 * cus ? 0.9 : 0.97);
       cb = best;
-      sort_items = cascs.empty() && items_of(cb) > cus;
+      // Longest first. (From six items per CU on it changes nothing in the mean over a binary16
+      // arena, 0.96-1.04x in 39 passes: those keep the list's order.)
+      const size_t items = items_of(cb);
+      sort_items = cascs.empty() && items > cus && (f32 || items < 6 * cus);
     }
   }
   // Each wave's page ids fit its 64 lanes: at most 64 blocks per wave.
@@ -1215,6 +1237,7 @@ int build_plan(yx_ctx* c, size_t window, size_t hq, size_t hkv, bool f32, size_t
   plan.slots = slot;
   plan.counters = subs.size();
   if (plan.items.size() > 0x7fffffff) return fail(YX_ERR_UNSUPPORTED, "too many work items");
+  c->decode_items = plan.items.size() * hkv;
   auto& p = c->plans[key];
   p = std::move(plan);
   p.cascades = cascs.size();
@@ -2111,6 +2134,8 @@ int yx_ctx_get_stat(yx_ctx* c, const char* key, uint64_t* out) {
     *out = c->split_tiles;
   else if (!std::strcmp(key, "prefill_plans"))
     *out = c->prefill_plans;
+  else if (!std::strcmp(key, "decode_items"))
+    *out = c->decode_items;
   else if (!std::strcmp(key, "matmul_kernel"))
     *out = c->mm_kernel;
   else if (!std::strcmp(key, "matmul_k_parts"))
