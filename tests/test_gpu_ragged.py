@@ -97,6 +97,7 @@ def _forks(batch, rows, ctx, prefix, page):
     (74, 7, 1250, 0, 16, 4, False, 296),       # shorter chunks estimated 1% better, 14% slower
     (134, 1, 1230, 0, 14, 2, False, 268),      # a few items beyond one round
     (22, 2, 2461, 2432, 40, 8, True, 352),     # f32 forks that read each other's pages
+    (60, 8, 3600, 0, 40, 8, False, None),      # whole prefill tiles in one round
 ])
 def test_work_lists_stay_whole_where_a_cut_does_not_pay(hip, batch, rows, ctx, prefix, hq, hkv, f32, items):
     """Passes that a longer or shorter chunk length made slower keep the plain split's items."""
