@@ -79,7 +79,7 @@ __device__ __forceinline__ void store_out4(float* out, uint32_t row, uint32_t co
 // was 4.8e-7 off 64 bits (2-norm), this is 1.8e-7, as that kernel.
 // With ks > 1 (grid y) the ks workgroups of a tile take consecutive stages and hand
 // their tiles over as matmul_bf16_rows does.
-// Measured (k = n = 2048): t 4096 739 -> 87 us (128 x 256 tiles, 395 TFLOP/s, 3x that in
+// Measured (k = n = 2048): t 4096 702 -> 81 us (128 x 256 tiles, 425 TFLOP/s, 3x that in
 // matrix instructions), t 2048 350 -> 54, t 512 90 -> 22, t 80 19.4 -> 12.0.
 template <int TM_, int TN_, int WM_, int WN_, int KU_, int kWaves_>
 struct MatmulTile {
@@ -351,7 +351,7 @@ __global__ __launch_bounds__(kMatmulThreads, T::kWavesPerSimd) void matmul_bf16_
 // partial tiles meet in LDS, nb tiles at a time in one of two halves (so one barrier per
 // nb tiles), and are added in wave order: the bits of matmul_bf16_rows without a split
 // of k. Grid: at most one workgroup per CU; workgroup i takes batches i, i + grid, ...
-// Measured (k 2048): 16 x 151936 240 -> 118 us (5.3 TB/s of w), 1 x 151936 128 -> 104,
+// Measured (k 2048): 16 x 151936 222 -> 120 us (5.2 TB/s of w), 1 x 151936 128 -> 104,
 // 16 x 16384 27 -> 15, 16 x 8192 14.9 -> 10.5; a third tile in flight or nontemporal
 // loads are 2-30% slower.
 static constexpr int kStreamWaves = 8;

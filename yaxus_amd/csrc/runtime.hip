@@ -1592,7 +1592,7 @@ int matmul_tiles_scratch(yx_ctx* c) {
 // shape's cost per stage (all CUs busy, measured over t 20-4096, k 1536-3072, n
 // 2000-151936) plus start and output, plus a split's hand-off (its last workgroup reads
 // ks partial tiles at about 50 GB/s). The estimate picks
-// the fastest or one within 5% of it in those shapes (t 4096, n 2048: 128 x 256 tiles 87
+// the fastest or one within 5% of it in those shapes (t 4096, n 2048: 128 x 256 tiles 87 (81 now)
 // us, 128 x 128 114, 64 x 128 123; t 512: 64 x 128 split in two 22.3, 128 x 128 in four
 // 22.9, 128 x 256 in two 45; t 80: 64 x 64 in four 12.0, 64 x 128 in eight 12.7).
 struct MatmulSplit {
